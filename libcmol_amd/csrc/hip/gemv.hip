@@ -193,25 +193,81 @@ int launch_gemv_b_finish(const GemvArgs &a, int epi, int splits, int ss_count, h
     return 0;
 }
 
-// Standalone operand preparation: one thread per (vector, block of 32).
-__global__ void k_act_prep(const float *__restrict__ x, int x_stride, int K, int n, ActOut o)
+// Standalone operand preparation: one thread per (vector, block of 32,
+// k-group), i.e. per 16-byte piece of the operand's high and low rows: two
+// 4-float loads, two 16-byte stores; the block's sum of squares meets over
+// the four k-group lanes.  Bound by its launch and one load-to-store round
+// trip (a 2048-input vector is 256 threads), then by the operand's bytes.
+// The earlier thread per 32-value block stored each half separately, 64
+// dependent 2-byte stores per thread: 13.2 us at 1 x 2048, now 2.0; 14.4 at
+// 32 x 2048, now 3.8.
+// VS: log2 of the vectors a wave covers.  The operand interleaves the
+// vectors per (block, k-group), so with 16 or more of them a wave takes 16
+// vectors of one block (512 contiguous bytes stored per k-group, whole
+// 128-byte lines read); with fewer, one vector of 16 blocks.
+// x and norm_w carry no alignment beyond a float's.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int VS>
+__global__ __launch_bounds__(256) void k_act_prep(const float *__restrict__ x, int x_stride, int K, int n, ActOut o)
 {
 #pragma clang fp contract(off)
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    const int v = blockIdx.y;
-    if (v >= n || b >= K / 32) return;
-    float ss = 0.0f;
-    for (int i = 0; i < 32; i++) {
-        const float xv = x[(size_t)v * x_stride + 32 * b + i];
-        ss += xv * xv;
-        act_put(o, v, 32 * b + i, xv);
+    const int l = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int g = l & 3;
+    const int v = blockIdx.y * (1 << VS) + ((l >> 2) & ((1 << VS) - 1));
+    const int b = ((blockIdx.x * 4 + wid) << (4 - VS)) + (l >> (2 + VS));
+    const bool act = v < n && b < K / 32;   // the four lanes of a block alike
+    // the k-group's inputs in operand order (the inverse of act_put's map):
+    // Q8_0 eight consecutive ones, the nibble formats 4g .. +3 and 16+4g ..
+    // +3, each four in the order 0, 2, 1, 3
+    const bool q8 = o.dt == DT_Q8_0;
+    const int k0 = 32 * b + (q8 ? 8 * g : 4 * g), k1 = k0 + (q8 ? 4 : 16);
+    float xv[8] = {}, wv[8];
+    if (act) {
+        const f4u a0 = *(const f4u *)(x + (size_t)v * x_stride + k0), a1 = *(const f4u *)(x + (size_t)v * x_stride + k1);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            xv[e] = a0[e];
+            xv[4 + e] = a1[e];
+        }
     }
-    if (o.ss) o.ss[(size_t)v * o.ss_stride + b] = ss;
+    if (o.norm_w && act) {
+        const f4u w0 = *(const f4u *)(o.norm_w + k0), w1 = *(const f4u *)(o.norm_w + k1);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            wv[e] = w0[e];
+            wv[4 + e] = w1[e];
+        }
+    }
+    float ss = 0.0f;
+    f16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        ss += xv[e] * xv[e];
+        const float t = (o.norm_w ? wv[e] * xv[e] : xv[e]) * ACT_SCALE;
+        const _Float16 h = (_Float16)t;
+        hi[e] = h;
+        lo[e] = (_Float16)((t - (float)h) * LO_SCALE);
+    }
+    if (!q8) {
+        hi = __builtin_shufflevector(hi, hi, 0, 2, 1, 3, 4, 6, 5, 7);
+        lo = __builtin_shufflevector(lo, lo, 0, 2, 1, 3, 4, 6, 5, 7);
+    }
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    if (!act) return;
+    f16x8 *dst = (f16x8 *)(o.q + (((size_t)b * 4 + g) * o.nrows + 2 * v) * 8);
+    dst[0] = hi;
+    dst[1] = lo;
+    if (o.ss && g == 0) o.ss[(size_t)v * o.ss_stride + b] = ss;
 }
 
 int launch_act_prep(const float *x, int x_stride, int K, int n, const ActOut &o, hipStream_t s)
 {
     const int nb = K / 32;
-    hipLaunchKernelGGL(k_act_prep, dim3((nb + 63) / 64, n), dim3(64), 0, s, x, x_stride, K, n, o);
+    if (n >= 16)
+        hipLaunchKernelGGL(k_act_prep<4>, dim3((nb + 3) / 4, (n + 15) / 16), dim3(256), 0, s, x, x_stride, K, n, o);
+    else
+        hipLaunchKernelGGL(k_act_prep<0>, dim3((nb + 63) / 64, n), dim3(256), 0, s, x, x_stride, K, n, o);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
