@@ -674,21 +674,24 @@ int launch_attn_prompt_dh(const AttnArgs &a, _Float16 *kv_hl, int last, hipStrea
 int launch_attn_prompt(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s)
 {
     const int G = a.n_heads / a.n_kv;
-    if (a.kv_f16 || G < 1 || G > 8 || a.n_heads % a.n_kv || a.n < 1 || (a.d_head != 64 && a.d_head != 128))
-        return -4;
-    if (a.split < 64 || a.split % KVT_POS || a.max_splits > ATT_MAX_MERGE) return -4;
-    if (!kv_hl || last < 1 || last > a.max_ctx) return -4;
+    if (G < 1 || G > 8 || a.n_heads % a.n_kv || a.n < 1 || (a.d_head != 64 && a.d_head != 128)) return -4;
+    if (a.split < 64 || a.split % 64 || a.max_splits > ATT_MAX_MERGE) return -4;
+    if ((!a.kv_f16 && !kv_hl) || last < 1 || last > a.max_ctx) return -4;
+    AttnArgs b = a;
     // the pass's split: the longest multiple of the planned one that still
     // gives every CU two work-groups (a 2048-token pass: one split, no
     // merge; 512-token passes: 256-512 positions).  Fewer splits than
     // planned always fit the partial buffers.
-    AttnArgs b = a;
     const long blocks = (long)a.n_kv * ((a.n + 64 / G - 1) / (64 / G));
     while (b.split * 2 <= a.max_ctx && blocks * ((last + 2 * b.split - 1) / (2 * b.split)) >= 2L * attn_cus())
         b.split *= 2;
     b.max_splits = (last + b.split - 1) / b.split;
-    const int rc = a.d_head == 128 ? launch_attn_prompt_dh<128>(b, kv_hl, last, s)
-                                   : launch_attn_prompt_dh<64>(b, kv_hl, last, s);
+    int rc;
+    if (a.kv_f16) {
+        rc = launch_attn_prompt16(b, s);
+    } else {
+        rc = a.d_head == 128 ? launch_attn_prompt_dh<128>(b, kv_hl, last, s) : launch_attn_prompt_dh<64>(b, kv_hl, last, s);
+    }
     if (rc) return rc;
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }

@@ -631,11 +631,11 @@ bool prompt_attn_on()
 }
 
 // Whether prompt passes of this model run the flash-style prompt attention
-// (fp32 cache, d_head 64 / 128, at most 8 query heads per kv head).
+// (d_head 64 / 128, at most 8 query heads per kv head).
 bool prompt_attn_fits(const cmolhip_hparams_t &h)
 {
     const int G = h.n_heads / h.n_kv_heads;
-    return prompt_attn_on() && !h.kv_f16 && (h.d_head == 64 || h.d_head == 128) && G >= 1 && G <= 8;
+    return prompt_attn_on() && (h.d_head == 64 || h.d_head == 128) && G >= 1 && G <= 8;
 }
 
 // Positions per attention work-group in a prompt pass: the split kernels
@@ -959,7 +959,7 @@ void plan_prefill(Plan &P, const cmolhip_model_desc_t *d)
     P.add((size_t)cap * np * 4);
     P.add((size_t)cap * np * h.d_head * 4);
     if (has_qk_norm(d)) P.add((size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head) * 4);
-    if (prompt_attn_fits(h)) P.add(attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx));
+    if (prompt_attn_fits(h) && !h.kv_f16) P.add(attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx));
     P.add(prefill_part_floats(h) * 4);
 }
 
@@ -1347,7 +1347,7 @@ int enqueue_prefill(cmolhip_model *m, Prefill &F, Batch &B, int n, bool last, hi
         at.out = nullptr;
         at.next = act_out(F.op_o, L.o.dtype, n, nullptr, nullptr, 0);
         // the pass's tokens share every K/V tile (flash style on MFMA); other
-        // shapes and fp16 caches take the split kernels
+        // shapes take the split kernels
         if (prompt_attn_on() && launch_attn_prompt(at, F.kv_hl, F.h_steps[3 * (n - 1) + 2], st) == 0) {
         } else {
             RC(launch_attn(at, st));
@@ -1478,7 +1478,7 @@ int build_prefill(cmolhip_model *m, Prefill &F)
     RC(arena_get(c, (size_t)cap * np, &F.pl));
     RC(arena_get(c, (size_t)cap * np * h.d_head, &F.po));
     if (m->qk_norm) RC(arena_get(c, (size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head), &F.qkv_raw));
-    if (prompt_attn_fits(h))
+    if (prompt_attn_fits(h) && !h.kv_f16)
         RC(arena_get(c, attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx) / sizeof(_Float16), &F.kv_hl));
     F.part_cap = prefill_part_floats(h);
     RC(arena_get(c, F.part_cap, &F.part));

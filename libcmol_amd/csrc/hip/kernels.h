@@ -302,12 +302,14 @@ int launch_attn_bal(const AttnArgs &a, hipStream_t s);   // a.bal > 0 (launch_at
 // prompt passes (the split layout of launch_attn).
 int launch_attn_merge_wave(const AttnArgs &a, hipStream_t s);
 // Prompt-pass attention (flash style on MFMA) for vectors that are
-// consecutive tokens of one session over an fp32 cache, d_head 64 / 128;
-// returns -4 for shapes it does not take (the caller runs launch_attn).
-// kv_hl: attn_prompt_kv_bytes of scratch for the high/low f16 copy of the
-// session's cache positions 0 .. last-1 (last = the pass's largest seqlen).
+// consecutive tokens of one session, d_head 64 / 128; returns -4 for shapes
+// it does not take (the caller runs launch_attn).  last = the pass's largest
+// seqlen.  kv_hl (fp32 caches only): attn_prompt_kv_bytes of scratch for the
+// high/low f16 copy of the session's cache positions 0 .. last-1.
 int launch_attn_prompt(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s);
 size_t attn_prompt_kv_bytes(int n_kv, int d_head, int max_ctx);
+// Its fp16-cache kernel and split merge.
+int launch_attn_prompt16(const AttnArgs &a, hipStream_t s);
 
 // QK-norm models (src/attn.c:62-101): the QKV matvec stores raw q|k|v rows;
 // this stage normalises each q and k head (RMSNorm over d_head, weights
