@@ -100,17 +100,181 @@ __device__ __forceinline__ void gemm_wload(const QTensor &w, uint32_t e, uint32_
     else h = 0u;
 }
 
+// RMSNorm factors of vectors m0 .. m0 + BM - 1 (past the last: its own) from
+// the producer's partial sums of squares, by NT threads into LDS: NT / BM
+// lanes per vector, eight partials in flight per lane.
+template <int BM, int NT>
+__device__ __forceinline__ void gemm_norms(const GemvArgs &a, int m0, float *s_nrm, int tid)
+{
+    constexpr int LPV = NT / BM;
+    static_assert(LPV >= 1 && LPV <= 64 && (LPV & (LPV - 1)) == 0, "lanes per vector");
+    const int vi = tid / LPV, sub = tid % LPV;
+    const float *p = a.in.ss + (size_t)min(m0 + vi, a.n - 1) * a.in.ss_stride;
+    float s = 0.0f;
+    for (int i0 = sub; i0 < a.in.ss_count; i0 += 8 * LPV) {
+        float q[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = i0 + k * LPV < a.in.ss_count ? p[i0 + k * LPV] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) s += q[k];
+    }
+    for (int o = LPV >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (sub == 0) s_nrm[vi] = 1.0f / sqrtf(s / (float)a.w.cols + a.in.eps);
+}
+
+// Operand piece (block b, k-group g) of vector v from its eight inputs in
+// natural order (the first four, then the second four: see piece_k): the
+// high and low rows' 16 bytes each.
+__device__ __forceinline__ void act_put8(const ActOut &o, int v, int b, int g, int k0, int k1, const f32x4 &x0,
+                                         const f32x4 &x1)
+{
+#pragma clang fp contract(off)
+    f16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float x = e < 4 ? x0[e] : x1[e - 4];
+        const float t = (o.norm_w ? o.norm_w[(e < 4 ? k0 : k1 - 4) + e] * x : x) * ACT_SCALE;
+        hi[e] = (_Float16)t;
+        lo[e] = (_Float16)((t - (float)hi[e]) * LO_SCALE);
+    }
+    if (o.dt != DT_Q8_0) {
+        hi = __builtin_shufflevector(hi, hi, 0, 2, 1, 3, 4, 6, 5, 7);
+        lo = __builtin_shufflevector(lo, lo, 0, 2, 1, 3, 4, 6, 5, 7);
+    }
+    f16x8 *dst = (f16x8 *)(o.q + (((size_t)b * 4 + g) * o.nrows + 2 * v) * 8);
+    dst[0] = hi;
+    dst[1] = lo;
+}
+
+// Epilogues of a tile of BM vectors x BR output rows (vectors m0 .., rows
+// r0 .., r0 a multiple of BR) by NT threads; src(vi, rl) gives the products of
+// vector m0 + vi and rows r0 + rl .. +3, scaled.  EPI_RESID and EPI_SWIGLU:
+// a thread per operand piece of the consumer (eight inputs, 32 contiguous
+// bytes for a vector's high and low rows), a wave over 16 vectors and the
+// block's four k-groups, so a k-group's stores are 512 contiguous bytes and
+// residual lines are used whole.  EPI_QKV: a thread per four rows (two RoPE
+// pairs), 16 lanes along a vector's rows.  The stores bound these epilogues:
+// one lane per row and 2-byte operand stores took 571 us for the gate/up
+// projection of 2048 tokens (22016 x 2048 Q4_0) where the same product with
+// plain stores takes 431; 479 with 16-byte ones (and gemm_norms).
+// Rows come in whole operand blocks (RESID, SWIGLU: the consumer's inputs)
+// or whole 16-row heads (QKV).
+template <int EPI, int BM, int BR, int NT, typename Src>
+__device__ __forceinline__ void epi_runs(const GemvArgs &a, Src src, int m0, int r0, int tid)
+{
+#pragma clang fp contract(off)
+    static_assert(BM % 16 == 0, "vectors per tile");
+    if constexpr (EPI == EPI_RESID || EPI == EPI_SWIGLU) {
+        constexpr int RPK = EPI == EPI_SWIGLU ? 2 : 1;   // rows per consumer input
+        constexpr int PV = BR / (8 * RPK);               // pieces per vector
+        static_assert(BR % (32 * RPK) == 0 && (BM * PV) % NT == 0, "whole blocks");
+        const bool q8 = a.next.dt == DT_Q8_0;
+#pragma unroll
+        for (int it = 0; it < BM * PV / NT; it++) {
+            const int i = tid + it * NT;
+            const int g = i & 3, vi = (i >> 2) % BM, bl = (i >> 2) / BM, v = m0 + vi;
+            const int b = r0 / RPK / 32 + bl;
+            const int o0 = q8 ? 8 * g : 4 * g, o1 = q8 ? o0 + 4 : o0 + 16;   // the piece's inputs in its block
+            const bool act = v < a.n && 32 * b * RPK < a.w.rows;
+            if constexpr (EPI == EPI_RESID) {
+                f32x4 x0 = {}, x1 = {};
+                if (act) {
+                    const size_t base = (size_t)v * a.out_stride + 32 * b;
+                    const float *res = (a.res ? a.res : a.out) + base;
+                    x0 = *(const f32x4 *)(res + o0) + src(vi, 32 * bl + o0);
+                    x1 = *(const f32x4 *)(res + o1) + src(vi, 32 * bl + o1);
+                    *(f32x4 *)(a.out + base + o0) = x0;
+                    *(f32x4 *)(a.out + base + o1) = x1;
+                    if (a.next.q) act_put8(a.next, v, b, g, 32 * b + o0, 32 * b + o1, x0, x1);
+                }
+                if (a.next.ss) {
+                    // sums of squares per 16 rows: Q8_0 lanes 0, 1 hold the
+                    // block's first 16 and lanes 2, 3 its second; otherwise
+                    // x0 belongs to the first and x1 to the second
+                    float s0 = x0[0] * x0[0] + x0[1] * x0[1] + x0[2] * x0[2] + x0[3] * x0[3];
+                    float s1 = x1[0] * x1[0] + x1[1] * x1[1] + x1[2] * x1[2] + x1[3] * x1[3];
+                    float *ss = a.next.ss + (size_t)v * a.next.ss_stride + 2 * b;
+                    if (q8) {
+                        s0 += s1;
+                        s0 += __shfl_xor(s0, 1, 64);
+                        if (act && !(g & 1)) ss[g >> 1] = s0;
+                    } else {
+                        s0 += __shfl_xor(s0, 1, 64);
+                        s0 += __shfl_xor(s0, 2, 64);
+                        s1 += __shfl_xor(s1, 1, 64);
+                        s1 += __shfl_xor(s1, 2, 64);
+                        if (act && g == 0) {
+                            ss[0] = s0;
+                            ss[1] = s1;
+                        }
+                    }
+                }
+            } else if (act) {
+                f32x4 hv[2];
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const int rl = 2 * (32 * bl + (p ? o1 : o0));
+                    const f32x4 ya = src(vi, rl), yb = src(vi, rl + 4);   // gate, up alternating
+                    hv[p][0] = (ya[0] / (1.0f + expf(-ya[0]))) * ya[1];
+                    hv[p][1] = (ya[2] / (1.0f + expf(-ya[2]))) * ya[3];
+                    hv[p][2] = (yb[0] / (1.0f + expf(-yb[0]))) * yb[1];
+                    hv[p][3] = (yb[2] / (1.0f + expf(-yb[2]))) * yb[3];
+                    if (a.out) *(f32x4 *)(a.out + (size_t)v * a.out_stride + 32 * b + (p ? o1 : o0)) = hv[p];
+                }
+                if (a.next.q) act_put8(a.next, v, b, g, 32 * b + o0, 32 * b + o1, hv[0], hv[1]);
+            }
+        }
+    } else {
+        static_assert(EPI == EPI_QKV && BR % 64 == 0 && (BM * BR / 4) % NT == 0, "whole rows");
+#pragma unroll
+        for (int it = 0; it < BM * BR / 4 / NT; it++) {
+            const int i = tid + it * NT;
+            const int vi = (i >> 4) % BM, rl = 64 * ((i >> 4) / BM) + 4 * (i & 15), v = m0 + vi;
+            if (v >= a.n || r0 + rl >= a.w.rows) continue;
+            const f32x4 y = src(vi, rl);
+            const int pos = epi_pos(a, v), row = r0 + rl + a.row_base;
+            const bool isq = row < a.nq, isk = !isq && row < a.nq + a.nkv;
+            const int rr = isq ? row : isk ? row - a.nq : row - a.nq - a.nkv;
+            const int h = rr / a.d_head, d = rr % a.d_head;
+            f32x4 x = y;
+            if (a.rope_on && (isq || isk)) {
+                const f32x4 cs = *(const f32x4 *)(a.rope + ((size_t)pos * (a.d_head / 2) + (d >> 1)) * 2);
+                x[0] = y[0] * cs[0] - y[1] * cs[1];
+                x[1] = y[0] * cs[1] + y[1] * cs[0];
+                x[2] = y[2] * cs[2] - y[3] * cs[3];
+                x[3] = y[2] * cs[3] + y[3] * cs[2];
+            }
+            if (isq) {
+                *(f32x4 *)(a.out + (size_t)v * a.out_stride + row) = x;
+                continue;
+            }
+            void *base = isk ? a.kv.k_base : a.kv.v_base;
+            const size_t o = kv_offset(a.kv, v) + ((size_t)h * a.max_ctx + pos) * a.d_head + d;
+            if (a.kv_f16)
+                *(f16x4 *)((_Float16 *)base + o) =
+                    f16x4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+            else *(f32x4 *)((float *)base + o) = x;
+        }
+    }
+}
+
 // WM wave rows of HG groups of 16 vectors each (GEMM_BM = 16 HG WM vectors
-// per work-group), four wave columns of 32 output rows: 4 WM waves
+// per work-group), four wave columns of 32 output rows: 4 WM waves.
+// Held to four waves per SIMD (128 VGPRs): the two work-groups that 64 KiB
+// of LDS allow need them.  Unheld, the Q8_0 and K-quant instances took
+// 129-160 VGPRs and ran one: 22016 x 2048 at 2048 vectors, Q8_0 590 -> 462 us,
+// Q4_K 822 -> 612 (4 VGPRs spilled), Q6_K 1031 -> 791 (18 spilled).
 template <int DT, int WM, int HG>
-__global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
+__global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(GemvArgs a, GemmShape sh)
 {
     constexpr int GEMM_BM = 16 * HG * WM, GEMM_WAVES = 4 * WM;
     constexpr int SEGS = GEMM_BM / 32;            // 64-row operand segments per (block, group)
     constexpr int PW = 16 * SEGS / GEMM_WAVES;    // operand copies per wave and stage
+    constexpr int NJ = 2, BN = GEMM_BN;           // virtual tiles per wave, output rows per work-group
     constexpr int ASTAGE = 4 * 4 * 2 * GEMM_BM * 16;   // [block][k-group][2 GEMM_BM rows][16 B]
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     uint8_t *s_a = smem;                                 // GEMM_STAGES x ASTAGE
+    static_assert(GEMM_BM * (BN + 4) * 4 <= GEMM_STAGES * ASTAGE, "epilogue tile");
 
     // XCD-aware tile order: work-groups b, b+8, b+16, ... share an XCD.  The
     // (vector tile, row tile) grid is cut into ga x (8 / ga) slices, one per
@@ -139,13 +303,7 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
     float nrm[HG][4] = {};
     if (a.in.ss) {
         float *s_nrm = (float *)(smem + (GEMM_STAGES - 1) * ASTAGE);
-        for (int vi = wid; vi < GEMM_BM; vi += GEMM_WAVES) {
-            const int v = min(m0 + vi, n - 1);
-            float s = 0.0f;
-            for (int i = l; i < a.in.ss_count; i += 64) s += a.in.ss[(size_t)v * a.in.ss_stride + i];
-            s = wave_sum(s);
-            if (l == 0) s_nrm[vi] = 1.0f / sqrtf(s / (float)a.w.cols + a.in.eps);
-        }
+        gemm_norms<GEMM_BM, GEMM_WAVES * 64>(a, m0, s_nrm, tid);
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < HG; h++)
@@ -156,10 +314,10 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
     // weight gather for this lane: virtual tile V -> (tile, column).  The
     // lane's element offsets within the tensor (32-bit: the host checks the
     // size) are fixed here; each quad adds a uniform part
-    uint32_t wq[2], wd[2];
+    uint32_t wq[NJ], wd[NJ];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int V = nt_ * 8 + wn * 2 + j;
+    for (int j = 0; j < NJ; j++) {
+        const int V = (nt_ * 4 + wn) * NJ + j;
         const int row = V * 16 + cl;
         const uint32_t wt = (uint32_t)min(row / R, a.w.row_tiles - 1), wc = (uint32_t)(row % R);
         wq[j] = wt * (uint32_t)BQ * 64u + wc + 16u * (uint32_t)g;   // cell * 64 + lane
@@ -175,9 +333,9 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
         arow[half] = 16u * (uint32_t)min(2 * m0 + 64 * half + (l & 32) + 2 * (l5 & 15) + (l5 >> 4), nrows - 1);
     }
 
-    u32x4 c0[GEMM_STAGES][2], c1[GEMM_STAGES][2];
-    typename QScale<DT>::T dv[GEMM_STAGES][2];
-    uint32_t hv[GEMM_STAGES][2];
+    u32x4 c0[GEMM_STAGES][NJ], c1[GEMM_STAGES][NJ];
+    typename QScale<DT>::T dv[GEMM_STAGES][NJ];
+    uint32_t hv[GEMM_STAGES][NJ];
     // loads of quad kk into stage st: 4 operand copies (of the tile's 32
     // 1 KiB pieces) and the codes/scales of the wave's two virtual tiles;
     // every load is issued unconditionally (padding blocks re-read a valid
@@ -199,16 +357,15 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
         const uint32_t uq = (uint32_t)(q * 64 + p * R);
         const uint32_t ud = is_kquant(DT) ? (uint32_t)(q * 16 + p * R) : (uint32_t)(q * 64 + 4 * p * R);
 #pragma unroll
-        for (int j = 0; j < 2; j++) gemm_wload<DT>(a.w, wq[j] + uq, wd[j] + ud, c0[st][j], c1[st][j], dv[st][j], hv[st][j]);
+        for (int j = 0; j < NJ; j++) gemm_wload<DT>(a.w, wq[j] + uq, wd[j] + ud, c0[st][j], c1[st][j], dv[st][j], hv[st][j]);
     };
 
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4 acc[HG][2];
+    f32x4 acc[HG][NJ];
 #pragma unroll
-    for (int h = 0; h < HG; h++) {
-        acc[h][0] = zero4;
-        acc[h][1] = zero4;
-    }
+    for (int h = 0; h < HG; h++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[h][j] = zero4;
 
     auto compute = [&](int st, int kk) {
         const int p = kk / BQ, q = kk - p * BQ;
@@ -217,10 +374,10 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
         const int nb = kk < ke ? min(4, nblk - (p * 4 * BQ + 4 * q)) : 0;
         const uint8_t *sa = s_a + st * ASTAGE;
         auto block = [&](int bi) {
-            f16x8 wv[2], wl[2];
-            BlockScale bs[2];
+            f16x8 wv[NJ], wl[NJ];
+            BlockScale bs[NJ];
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < NJ; j++) {
                 wv[j] = deq_block<DT>(c0[st][j], c1[st][j], hv[st][j], bi);
                 wl[j] = wv[j] * (_Float16)LO_INV_SCALE;
                 bs[j] = block_scale<DT>(dv[st][j], bi);
@@ -231,7 +388,7 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
                 const f16x8 xh = *(const f16x8 *)row;
                 const f16x8 xl = *(const f16x8 *)(row + 16 * 16);
 #pragma unroll
-                for (int j = 0; j < 2; j++) mfma_block_hl<DT>(acc[h][j], xh, xl, wv[j], wl[j], bs[j]);
+                for (int j = 0; j < NJ; j++) mfma_block_hl<DT>(acc[h][j], xh, xl, wv[j], wl[j], bs[j]);
             }
         };
         // a whole quad is one straight run (the four blocks' loads, MFMA
@@ -274,35 +431,38 @@ __global__ __launch_bounds__(4 * WM * 64) void k_gemm(GemvArgs a, GemmShape sh)
     __syncthreads();
 
     // lane l holds, per vector group h and tile j, output row 16V + cl for
-    // vectors m0 + 16 HG wm + 16h + 4(l>>4) + {0, 1, 2, 3}
+    // vectors m0 + 16 HG wm + 16h + 4(l>>4) + {0, 1, 2, 3}.  Plain and partial
+    // sums leave from here (64-byte runs of a vector's rows); the other
+    // epilogues take the tile through LDS, 16 bytes at a time
+    const bool direct = sh.ks > 1 || sh.epi == EPI_STORE;
+    float *tile = (float *)smem;
 #pragma unroll
     for (int h = 0; h < HG; h++) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int V = nt_ * 8 + wn * 2 + j;
+        for (int j = 0; j < NJ; j++) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int vi = 16 * HG * wm + 16 * h + 4 * (l >> 4) + e;
-                const int v = m0 + vi;
-                const bool act = v < n;
+                const int rl = (wn * NJ + j) * 16 + cl, row = nt_ * BN + rl;
+                const int vi = 16 * HG * wm + 16 * h + 4 * (l >> 4) + e, v = m0 + vi;
                 float y = acc[h][j][e] * ACT_INV_SCALE;
-                if (sh.ks > 1) {
-                    // this k range's partial sum (the finish kernel adds the
-                    // ranges in order, then scales and runs the epilogue)
-                    const int row = V * 16 + cl;
-                    if (act && row < a.w.rows) a.part[((size_t)blockIdx.y * n + v) * a.w.rows + row] = y;
-                    continue;
-                }
-                if (a.in.ss) y *= nrm[h][e];
-                const int vv = act ? v : 0;
-                switch (sh.epi) {
-                case EPI_STORE: epilogue<EPI_STORE>(a, V, cl, 16, vv, act, y); break;
-                case EPI_RESID: epilogue<EPI_RESID>(a, V, cl, 16, vv, act, y); break;
-                case EPI_SWIGLU: epilogue<EPI_SWIGLU>(a, V, cl, 16, vv, act, y); break;
-                default: epilogue<EPI_QKV>(a, V, cl, 16, vv, act, y); break;
+                // partial sums of a k range: the finish kernel adds the
+                // ranges in order, then scales and runs the epilogue
+                if (a.in.ss && sh.ks == 1) y *= nrm[h][e];
+                if (!direct) tile[vi * (BN + 4) + rl] = y;
+                else if (v < n && row < a.w.rows) {
+                    if (sh.ks > 1) a.part[((size_t)blockIdx.y * n + v) * a.w.rows + row] = y;
+                    else a.out[(size_t)v * a.out_stride + row] = y;
                 }
             }
         }
+    }
+    if (direct) return;
+    __syncthreads();
+    auto src = [&](int vi, int rl) { return *(const f32x4 *)&tile[vi * (BN + 4) + rl]; };
+    switch (sh.epi) {
+    case EPI_RESID: epi_runs<EPI_RESID, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
+    case EPI_SWIGLU: epi_runs<EPI_SWIGLU, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
+    default: epi_runs<EPI_QKV, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
     }
 }
 
