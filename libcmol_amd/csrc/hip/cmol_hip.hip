@@ -341,6 +341,17 @@ int cmolhip_gemm_prepared(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, const vo
 
 } // extern "C"
 
+// Partial-sum floats a product of n vectors takes when given room, and what
+// it insists on.
+static size_t product_part_floats(const cmolhip_qtensor_t &w, int n)
+{
+    return n <= 32 ? gemv_part_floats(to_qt(w), n) : gemm_part_floats(to_qt(w), n);
+}
+static size_t product_part_least(const cmolhip_qtensor_t &w, int n)
+{
+    return n <= 32 ? gemv_part_floats(to_qt(w), n) : gemm_part_least(to_qt(w), n);
+}
+
 // dy[n][rows] = W . op for a prepared operand: up to 32 vectors stream the
 // weights once through the matvec (k-split partial sums in part, part_cap
 // floats), more run the tiled MFMA GEMM.
@@ -376,9 +387,14 @@ int cmolhip_gemm_prepared_timed(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, co
     // the arena space of k-split partial sums is released at once: later
     // work on this stream runs after the kernels
     const size_t mark = arena_mark(c);
-    const size_t pf = n <= 32 ? gemv_part_floats(to_qt(*w), n) : gemm_part_floats(to_qt(*w), n);
+    const size_t least = product_part_least(*w, n);
+    size_t pf = std::max(least, product_part_floats(*w, n));
     float *part = nullptr;
     int rc = pf ? arena_get(c, pf, &part) : E_OK;
+    if (rc == E_OOM && least < pf) {   // a small arena: fewer k ranges
+        pf = least;
+        rc = pf ? arena_get(c, pf, &part) : E_OK;
+    }
     if (rc == E_OK) rc = launch_product(c, w, op, n, ss, eps, dy, part, pf, ev_start, ev_stop);
     arena_release(c, mark);
     return rc;
@@ -413,8 +429,9 @@ int cmolhip_gemm_noalloc(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, const flo
     // scratch layout: operand | sum-of-squares partials | k-split partial sums
     const size_t op_b = align_up(act_bytes(w->cols, n), ALIGN);
     const size_t ss_b = norm_w ? align_up((size_t)n * (w->cols / 32) * 4, ALIGN) : 0;
-    const size_t pf = n <= 32 ? gemv_part_floats(to_qt(*w), n) : gemm_part_floats(to_qt(*w), n);
-    if (op_b + ss_b + pf * 4 > NOALLOC_SCRATCH_BYTES) return E_ARGS;   // beyond the fixed scratch
+    const size_t least = product_part_least(*w, n);
+    if (op_b + ss_b + least * 4 > NOALLOC_SCRATCH_BYTES) return E_ARGS;   // beyond the fixed scratch
+    const size_t pf = std::min(std::max(least, product_part_floats(*w, n)), (NOALLOC_SCRATCH_BYTES - op_b - ss_b) / 4);
     float *ss = norm_w ? (float *)(base + op_b) : nullptr;
     float *part = pf ? (float *)(base + op_b + ss_b) : nullptr;
     RC(cmolhip_act_prepare(c, dx, n, w->cols, w->dtype, norm_w, base, ss));
@@ -929,12 +946,29 @@ void plan_batch(Plan &P, const cmolhip_model_desc_t *d, int cap, int ms)
     if (has_qk_norm(d)) P.add((size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head) * 4);
 }
 
-// Partial sums a prompt pass's split-K GEMMs may need: GEMM_KS_MAX ranges of
-// the pass's tokens for the widest of q|k|v and the d_model-row matrices.
-size_t prefill_part_floats(const cmolhip_hparams_t &h)
+// Partial sums the split-K GEMMs of a prompt pass of up to prefill_chunk
+// tokens need: the largest over the layers' matrices and pass lengths (whole
+// 32-vector tiles and the full pass: the split depends on the tile count).
+size_t prefill_part_floats(const cmolhip_model_desc_t *d)
 {
-    const size_t rows = (size_t)h.d_model + 2 * (size_t)h.n_kv_heads * h.d_head;
-    return (size_t)GEMM_KS_MAX * prefill_cap(h) * rows;
+    const cmolhip_hparams_t &h = d->hp;
+    const int cap = prefill_cap(h);
+    size_t m = 0;
+    auto need = [&](int rows, int cols) {
+        const QTensor t = shape_qt(DT_Q4_0, rows, cols, layer_fold(d, rows, cols));
+        for (int n = 32; n < cap + 32; n += 32) m = std::max(m, gemm_part_floats(t, std::min(n, cap)));
+    };
+    const int kvd = h.n_kv_heads * h.d_head;
+    for (int l = 0; l < h.n_layers; l++) {
+        const QkvRuns R = qkv_runs(d->layers[l], h);
+        for (int r = 0; r < R.n; r++)
+            if (l == 0 || R.n > 1) need(R.rows[r], h.d_model);
+    }
+    need(h.d_model + 2 * kvd, h.d_model);
+    need(h.d_model, h.d_model);
+    need(2 * h.d_ffn, h.d_model);
+    need(h.d_model, h.d_ffn);
+    return m;
 }
 
 // Buffers of the prompt pass, in allocation order (mirrored by build_prefill).
@@ -960,7 +994,7 @@ void plan_prefill(Plan &P, const cmolhip_model_desc_t *d)
     P.add((size_t)cap * np * h.d_head * 4);
     if (has_qk_norm(d)) P.add((size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head) * 4);
     if (prompt_attn_fits(h) && !h.kv_f16) P.add(attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx));
-    P.add(prefill_part_floats(h) * 4);
+    P.add(prefill_part_floats(d) * 4);
 }
 
 
@@ -1456,7 +1490,7 @@ int build_batch(cmolhip_model *m, Batch &B, int cap, size_t part_floats)
     return E_OK;
 }
 
-int build_prefill(cmolhip_model *m, Prefill &F)
+int build_prefill(cmolhip_model *m, Prefill &F, size_t part_floats)
 {
     cmolhip_ctx_t *c = m->ctx;
     const cmolhip_hparams_t &h = m->hp;
@@ -1480,8 +1514,8 @@ int build_prefill(cmolhip_model *m, Prefill &F)
     if (m->qk_norm) RC(arena_get(c, (size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head), &F.qkv_raw));
     if (prompt_attn_fits(h) && !h.kv_f16)
         RC(arena_get(c, attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx) / sizeof(_Float16), &F.kv_hl));
-    F.part_cap = prefill_part_floats(h);
-    RC(arena_get(c, F.part_cap, &F.part));
+    F.part_cap = part_floats;
+    if (part_floats) RC(arena_get(c, part_floats, &F.part));
     HC(hipHostMalloc((void **)&F.h_steps, (size_t)cap * 3 * 4, hipHostMallocDefault));
     HC(hipHostMalloc((void **)&F.h_slots, (size_t)cap * 4, hipHostMallocDefault));
     return E_OK;
@@ -1742,7 +1776,7 @@ int build_model(cmolhip_model *m, const cmolhip_model_desc_t *d, const Plan &P)
     m->multi.reset(new Batch());
     RC(build_batch(m, *m->multi, multi_cap(h), batch_part_floats(d, multi_cap(h))));
     m->pf.reset(new Prefill());
-    RC(build_prefill(m, *m->pf));
+    RC(build_prefill(m, *m->pf, prefill_part_floats(d)));
     if (persist_format(d)) RC(build_persist(m, persist_format(d)));
     HC(hipStreamSynchronize(c->stream));
     if (m->use_graph) {

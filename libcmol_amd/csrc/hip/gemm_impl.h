@@ -3,16 +3,19 @@
 // format by gemm_q4.hip / gemm_q5.hip / gemm_q8.hip / gemm_q4k.hip /
 // gemm_q6k.hip.
 //
-// One work-group computes a 64-vector x 128-row output tile (32 x 128 with
-// four waves where 64-vector tiles would leave half the CUs idle).  Its
-// eight waves form a 2 x 4 grid: wave (wm, wn) owns vectors 32wm..32wm+31
-// (two groups of 16, each with a 16-row high and a 16-row low operand block
-// in LDS) and output rows 32wn..32wn+31 (two 16-row "virtual tiles").  The
-// k loop walks block quads through a two-stage pipeline: the activation
-// operand of quad kk+1 is copied into LDS with direct-to-LDS loads and each
-// wave loads the weight codes of its two virtual tiles for it into
-// registers while quad kk is contracted.  Two stages (64 KiB of LDS) keep two work-groups on a CU,
-// which hides more latency than a third stage in flight with one.
+// One work-group of four waves computes a 32-vector x 128-row output tile:
+// its vectors are two groups of 16, each with a 16-row high and a 16-row low
+// operand block in LDS, and wave w owns output rows 32w .. 32w+31 (two 16-row
+// "virtual tiles").  The k loop walks block quads through a two-stage
+// pipeline: the activation operand of quad kk+1 is copied into LDS with
+// direct-to-LDS loads and each wave loads the weight codes of its two
+// virtual tiles for it into registers while quad kk is contracted.  32 KiB
+// of LDS and 128 VGPRs keep four work-groups on a CU, each with its own
+// barrier.  Eight-wave 64 x 128 tiles (two work-groups per CU, half the weight
+// decoding per product) took, Q4_0 11008 inputs x 2048 rows / 2048 x 22016:
+// 2048 vectors 211 / 417 us against 216 / 406, 1500 vectors 192 / 321 against
+// 170 / 315, 512 vectors 67 / 126 (k split) against 66 / 119, and at 128
+// vectors or fewer up to 40 % longer.
 // Weights of any fold are read in place: virtual tile V of part p gathers,
 // for column c', the codes of row 16V + c' from tile (16V + c') / R,
 // column p*R + c' % R.
@@ -26,6 +29,12 @@
 #pragma once
 #include "gemv_impl.h"
 
+// Adds the ks k ranges' partial sums of a prompt GEMM in order, applies the
+// RMSNorm factor and runs the epilogue (gemv.hip).
+int launch_gemm_finish(const GemvArgs &a, int epi, int ks, hipStream_t s);
+
+#define GEMM_NT 256   // threads per work-group
+#define GEMM_BM 32    // vectors per work-group
 #define GEMM_BN 128   // output rows per work-group (8 virtual tiles)
 #define GEMM_STAGES 2 // quads in flight
 
@@ -33,10 +42,10 @@ struct GemmShape {
     int epi;
     int mt;          // vector tiles (GEMM_BM vectors each)
     int nt;          // 128-row tiles
-    int vt;          // 16-row virtual tiles (ceil(rows / 16))
     int ga;          // XCD slices along the vector tiles (1, 2, 4, 8)
     int mts, nts;    // vector / row tiles per slice
     int ks, kq;      // k ranges (grid.y) of kq block quads each; ks > 1: fp32 partial sums to a.part
+    int fq;          // > 0: after fq quads (even) of its range a work-group sets its sums aside in LDS
 };
 
 // acc += the block's contribution for 16 vectors: xh holds their high
@@ -258,20 +267,18 @@ __device__ __forceinline__ void epi_runs(const GemvArgs &a, Src src, int m0, int
     }
 }
 
-// WM wave rows of HG groups of 16 vectors each (GEMM_BM = 16 HG WM vectors
-// per work-group), four wave columns of 32 output rows: 4 WM waves.
-// Held to four waves per SIMD (128 VGPRs): the two work-groups that 64 KiB
-// of LDS allow need them.  Unheld, the Q8_0 and K-quant instances took
-// 129-160 VGPRs and ran one: 22016 x 2048 at 2048 vectors, Q8_0 590 -> 462 us,
-// Q4_K 822 -> 612 (4 VGPRs spilled), Q6_K 1031 -> 791 (18 spilled).
-template <int DT, int WM, int HG>
-__global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(GemvArgs a, GemmShape sh)
+// Held to four waves per SIMD (128 VGPRs).  Unheld, the Q8_0 and K-quant
+// instances took 129-160 and ran half the work-groups: 22016 x 2048 at 2048
+// vectors, Q8_0 590 -> 462 us, Q4_K 822 -> 612 (4 VGPRs spilled), Q6_K 1031
+// -> 791 (14 spilled).
+template <int DT>
+__global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(GemvArgs a, GemmShape sh)
 {
-    constexpr int GEMM_BM = 16 * HG * WM, GEMM_WAVES = 4 * WM;
-    constexpr int SEGS = GEMM_BM / 32;            // 64-row operand segments per (block, group)
-    constexpr int PW = 16 * SEGS / GEMM_WAVES;    // operand copies per wave and stage
-    constexpr int NJ = 2, BN = GEMM_BN;           // virtual tiles per wave, output rows per work-group
+    constexpr int HG = 2, NJ = 2;                 // vector groups and virtual tiles per wave
+    constexpr int PW = 16 / (GEMM_NT / 64);       // 64-row operand copies per wave and stage
     constexpr int ASTAGE = 4 * 4 * 2 * GEMM_BM * 16;   // [block][k-group][2 GEMM_BM rows][16 B]
+    constexpr int BN = GEMM_BN;
+    static_assert(GEMM_BM == 16 * HG && GEMM_BN == 16 * NJ * (GEMM_NT / 64), "tile");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     uint8_t *s_a = smem;                                 // GEMM_STAGES x ASTAGE
     static_assert(GEMM_BM * (BN + 4) * 4 <= GEMM_STAGES * ASTAGE, "epilogue tile");
@@ -288,7 +295,6 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
 
     const int tid = threadIdx.x, l = tid & 63, g = l >> 4, cl = l & 15;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wid % WM, wn = wid / WM;
     const int n = a.n, nrows = 2 * n;
     const int BQ = a.w.block_quads, F = a.w.fold, R = 16 / F;
     const int nblk = a.w.cols >> 5;
@@ -299,16 +305,16 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     // RMSNorm scales of the tile's vectors from the producer's partials,
     // passed through the last stage's LDS (untouched until the k loop's
     // first copy into it, which follows a wait and a barrier) to the lanes
-    // that apply them: lane l's vectors 16 HG wm + 16h + 4(l>>4) + e
+    // that apply them: lane l's vectors 16h + 4(l>>4) + e
     float nrm[HG][4] = {};
     if (a.in.ss) {
         float *s_nrm = (float *)(smem + (GEMM_STAGES - 1) * ASTAGE);
-        gemm_norms<GEMM_BM, GEMM_WAVES * 64>(a, m0, s_nrm, tid);
+        gemm_norms<GEMM_BM, GEMM_NT>(a, m0, s_nrm, tid);
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < HG; h++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) nrm[h][e] = s_nrm[16 * HG * wm + 16 * h + 4 * (l >> 4) + e];
+            for (int e = 0; e < 4; e++) nrm[h][e] = s_nrm[16 * h + 4 * (l >> 4) + e];
     }
 
     // weight gather for this lane: virtual tile V -> (tile, column).  The
@@ -317,21 +323,17 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     uint32_t wq[NJ], wd[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const int V = (nt_ * 4 + wn) * NJ + j;
+        const int V = (nt_ * 4 + wid) * NJ + j;
         const int row = V * 16 + cl;
         const uint32_t wt = (uint32_t)min(row / R, a.w.row_tiles - 1), wc = (uint32_t)(row % R);
         wq[j] = wt * (uint32_t)BQ * 64u + wc + 16u * (uint32_t)g;   // cell * 64 + lane
         wd[j] = is_kquant(DT) ? wt * (uint32_t)BQ * 16u + wc : wt * (uint32_t)BQ * 64u + 4u * wc;
     }
-    // operand rows of this lane's two 64-row halves (LDS rows of each 32-row
-    // group: the 16 high parts, then the 16 low parts of its 16 vectors,
-    // operand rows 2v and 2v+1)
-    uint32_t arow[SEGS];
-#pragma unroll
-    for (int half = 0; half < SEGS; half++) {
-        const int l5 = l & 31;
-        arow[half] = 16u * (uint32_t)min(2 * m0 + 64 * half + (l & 32) + 2 * (l5 & 15) + (l5 >> 4), nrows - 1);
-    }
+    // operand row of this lane's copies (LDS rows of each 32-row group: the 16
+    // high parts, then the 16 low parts of its 16 vectors, operand rows 2v and
+    // 2v+1)
+    const int l5 = l & 31;
+    const uint32_t arow = 16u * (uint32_t)min(2 * m0 + (l & 32) + 2 * (l5 & 15) + (l5 >> 4), nrows - 1);
 
     u32x4 c0[GEMM_STAGES][NJ], c1[GEMM_STAGES][NJ];
     typename QScale<DT>::T dv[GEMM_STAGES][NJ];
@@ -346,12 +348,10 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
         const int b0 = p * 4 * BQ + 4 * q;
 #pragma unroll
         for (int i = 0; i < PW; i++) {
-            const int s = wid * PW + i;           // 16 (block, group) pairs x SEGS segments
-            const int seg = s / SEGS, half = i % SEGS;   // wid * PW % SEGS == 0
-            const int bi = seg >> 2, gg = seg & 3;
+            const int s = wid * PW + i, bi = s >> 2, gg = s & 3;   // (block, k-group)
             const int blk = min(b0 + bi, nblk - 1);
-            const uint8_t *src = (const uint8_t *)a.in.q + ((size_t)blk * 4 + gg) * nrows * 16 + arow[half];
-            uint8_t *dst = s_a + st * ASTAGE + ((bi * 4 + gg) * 2 * GEMM_BM + 64 * half) * 16;
+            const uint8_t *src = (const uint8_t *)a.in.q + ((size_t)blk * 4 + gg) * nrows * 16 + arow;
+            uint8_t *dst = s_a + st * ASTAGE + s * 2 * GEMM_BM * 16;
             __builtin_amdgcn_global_load_lds((const gvoid_t *)src, (lvoid_t *)dst, 16, 0, 0);
         }
         const uint32_t uq = (uint32_t)(q * 64 + p * R);
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
             }
 #pragma unroll
             for (int h = 0; h < HG; h++) {
-                const uint8_t *row = &sa[((bi * 4 + g) * 2 * GEMM_BM + 32 * HG * wm + 32 * h + cl) * 16];
+                const uint8_t *row = &sa[((bi * 4 + g) * 2 * GEMM_BM + 32 * h + cl) * 16];
                 const f16x8 xh = *(const f16x8 *)row;
                 const f16x8 xl = *(const f16x8 *)(row + 16 * 16);
 #pragma unroll
@@ -414,7 +414,18 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     __builtin_amdgcn_sched_barrier(0);
     // the body is unconditional (steps past the end compute nothing and
     // re-read the last quad) so every wait count is the same on each pass
+    const bool halves = sh.fq && kb + sh.fq < ke;
+    f32x4 *aside = (f32x4 *)(smem + GEMM_STAGES * ASTAGE) + tid;   // [HG NJ][threads], each thread its own
     for (int k0 = kb; k0 < ke; k0 += GEMM_STAGES) {
+        if (halves && k0 == kb + sh.fq) {
+#pragma unroll
+            for (int h = 0; h < HG; h++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    aside[(h * NJ + j) * GEMM_NT] = acc[h][j];
+                    acc[h][j] = zero4;
+                }
+        }
 #pragma unroll
         for (int u = 0; u < GEMM_STAGES; u++) {
             const int kk = k0 + u;
@@ -431,7 +442,7 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     __syncthreads();
 
     // lane l holds, per vector group h and tile j, output row 16V + cl for
-    // vectors m0 + 16 HG wm + 16h + 4(l>>4) + {0, 1, 2, 3}.  Plain and partial
+    // vectors m0 + 16h + 4(l>>4) + {0, 1, 2, 3}.  Plain and partial
     // sums leave from here (64-byte runs of a vector's rows); the other
     // epilogues take the tile through LDS, 16 bytes at a time
     const bool direct = sh.ks > 1 || sh.epi == EPI_STORE;
@@ -440,10 +451,11 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     for (int h = 0; h < HG; h++) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
+            if (halves) acc[h][j] += aside[(h * NJ + j) * GEMM_NT];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int rl = (wn * NJ + j) * 16 + cl, row = nt_ * BN + rl;
-                const int vi = 16 * HG * wm + 16 * h + 4 * (l >> 4) + e, v = m0 + vi;
+                const int rl = (wid * NJ + j) * 16 + cl, row = nt_ * BN + rl;
+                const int vi = 16 * h + 4 * (l >> 4) + e, v = m0 + vi;
                 float y = acc[h][j][e] * ACT_INV_SCALE;
                 // partial sums of a k range: the finish kernel adds the
                 // ranges in order, then scales and runs the epilogue
@@ -460,86 +472,76 @@ __global__ __launch_bounds__(4 * WM * 64) __attribute__((amdgpu_waves_per_eu(4))
     __syncthreads();
     auto src = [&](int vi, int rl) { return *(const f32x4 *)&tile[vi * (BN + 4) + rl]; };
     switch (sh.epi) {
-    case EPI_RESID: epi_runs<EPI_RESID, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
-    case EPI_SWIGLU: epi_runs<EPI_SWIGLU, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
-    default: epi_runs<EPI_QKV, GEMM_BM, BN, GEMM_WAVES * 64>(a, src, m0, nt_ * BN, tid); break;
+    case EPI_RESID: epi_runs<EPI_RESID, GEMM_BM, BN, GEMM_NT>(a, src, m0, nt_ * BN, tid); break;
+    case EPI_SWIGLU: epi_runs<EPI_SWIGLU, GEMM_BM, BN, GEMM_NT>(a, src, m0, nt_ * BN, tid); break;
+    default: epi_runs<EPI_QKV, GEMM_BM, BN, GEMM_NT>(a, src, m0, nt_ * BN, tid); break;
     }
 }
 
-template <int DT, int WM, int HG>
-int launch_gemm_wm(const GemvArgs &a, int epi, hipStream_t s, int ks = 1)
-{
-    constexpr int BM = 16 * HG * WM;
-    GemmShape sh;
-    sh.epi = epi;
-    const int KQ = a.w.fold * a.w.block_quads;
-    sh.ks = ks;
-    sh.kq = (KQ + ks - 1) / ks;
-    if (ks > 1 && (!a.part || (size_t)ks * a.n * a.w.rows > a.part_cap)) return -6;
-    sh.mt = (a.n + BM - 1) / BM;
-    sh.vt = (a.w.rows + 15) / 16;
-    sh.nt = (sh.vt + 7) / 8;
-    // one slice of vector tiles per XCD (at M = 2048: 512 KiB of operand
-    // per 64-vector tile, four per XCD) unless there are fewer vector tiles
-    sh.ga = 8;
-    while (sh.ga > 1 && sh.ga > sh.mt) sh.ga >>= 1;
-    sh.mts = (sh.mt + sh.ga - 1) / sh.ga;
-    sh.nts = (sh.nt + 8 / sh.ga - 1) / (8 / sh.ga);
-    const long wgs = 8L * sh.mts * sh.nts;
-    if (wgs > 0x7fffffffL) return -6;
-    const size_t lds = (size_t)GEMM_STAGES * 4 * 4 * 2 * BM * 16;
-    const dim3 grid((unsigned)wgs, (unsigned)ks);
-    if (a.ev_start)
-        hipExtLaunchKernelGGL((k_gemm<DT, WM, HG>), grid, dim3(4 * WM * 64), lds, s, a.ev_start,
-                              ks > 1 ? nullptr : a.ev_stop, 0, a, sh);
-    else
-        hipLaunchKernelGGL((k_gemm<DT, WM, HG>), grid, dim3(4 * WM * 64), lds, s, a, sh);
-    if (ks > 1) return launch_gemv_b_finish(a, epi, ks, a.in.ss ? a.in.ss_count : 0, s);
-    return 0;
-}
-
-// k ranges of the split-K prompt GEMM: the fewest (a power of two, at most
-// GEMM_KS_MAX) that give the 64-vector tiles two work-groups per CU, each
-// range at least 8 block quads, within the partial-sum buffer; 1 when the
-// tiles already fill the chip or no buffer is given.  CMOL_GEMM_KSPLIT=0
-// turns it off (measurements).
+// k ranges of the prompt GEMM.  The tiles of a narrow matrix or a short
+// prompt leave CUs idle, and every work-group walks its k range at the
+// latency of a step (about 1.2 us per block quad), so the ranges are doubled
+// while the grid still fits one work-group per CU (two block quads or more
+// each), and further, up to four per CU, while they keep ten quads.  Each range
+// costs a write and a read of its partial sums in the finish kernel, which
+// is why short ranges stop at one per CU: Q4_0, with finish, 64 vectors:
+// 2048 x 2048 18.2 us in one range, 11.6 / 11.4 in 4 / 8 (taken), 14.6 in 16;
+// 2048 x 11008 76, 26.8 in 4, 19.5 in 8 (taken), 19.7 in 16; 22016 x 2048 28.1
+// in one (taken), 27.5 in 2, 30.1 in 4.  At 512 vectors 2048 x 2048 20.2 in
+// one (taken), 23.9 in 2; 2048 x 11008 82.9, 72.6 in 2, 66.1 in 4 (taken).
+// Within the partial-sum buffer (part_cap floats).  CMOL_GEMM_KSPLIT=0 turns
+// it off (measurements).
 static inline int gemm_ks(const QTensor &w, int n, size_t part_cap)
 {
     static const bool on = [] {
         const char *e = getenv("CMOL_GEMM_KSPLIT");
         return !(e && e[0] == '0');
     }();
-    const long tiles64 = (long)((n + 63) / 64) * (((w.rows + 15) / 16 + 7) / 8);
+    if (!on) return 1;
+    const long tiles = (long)((n + GEMM_BM - 1) / GEMM_BM) * ((w.rows + GEMM_BN - 1) / GEMM_BN);
     const int KQ = w.fold * w.block_quads;
     int ks = 1;
-    if (!on) return 1;
-    while (ks < GEMM_KS_MAX && tiles64 * ks < 2L * gemv_cus() && KQ / (2 * ks) >= 8 &&
-           (size_t)(2 * ks) * n * w.rows <= part_cap)
+    while (ks < GEMM_KS_MAX && (size_t)(2 * ks) * n * w.rows <= part_cap &&
+           ((tiles * 2 * ks <= gemv_cus() && KQ / (2 * ks) >= 2) ||
+            (tiles * 2 * ks <= 4L * gemv_cus() && KQ / (2 * ks) >= 10)))
         ks *= 2;
     return ks;
 }
 
-static inline int gemm_ksplit(const GemvArgs &a, long)
-{
-    return a.part ? gemm_ks(a.w, a.n, a.part_cap) : 1;
-}
-
-// 64-vector work-groups (two per CU) unless their tiles cover at most half
-// the CUs (2048 output rows at 512 tokens: 128 tiles); then 32-vector ones
-// (five per CU), twice as many.  Four-wave 64-vector work-groups (four
-// vector groups per wave: fewer decode and address instructions per
-// product, 140 VGPRs, two waves per SIMD) ran 10-15 % slower at 2048 tokens:
-// the kernel needs the waves to hide latency more than it needs fewer
-// instructions.
 template <int DT>
 int launch_gemm_dt(const GemvArgs &a, int epi, hipStream_t s)
 {
     if (epi < EPI_STORE || epi > EPI_QKV) return -6;
     // the kernel's per-lane weight offsets are 32-bit
     if ((size_t)a.w.row_tiles * a.w.block_quads * 64 * QFmt<DT>::LANE_BYTES > 0xffffffffUL) return -6;
-    const long tiles64 = (long)((a.n + 63) / 64) * (((a.w.rows + 15) / 16 + 7) / 8);
-    const int ks = gemm_ksplit(a, tiles64);
-    if (ks > 1) return launch_gemm_wm<DT, 2, 2>(a, epi, s, ks);
-    if (tiles64 <= gemv_cus() / 2) return launch_gemm_wm<DT, 1, 2>(a, epi, s);
-    return launch_gemm_wm<DT, 2, 2>(a, epi, s);
+    GemmShape sh;
+    sh.epi = epi;
+    const int KQ = a.w.fold * a.w.block_quads;
+    const int ks = a.part ? gemm_ks(a.w, a.n, a.part_cap) : 1;
+    sh.ks = ks;
+    sh.kq = (KQ + ks - 1) / ks;
+    sh.mt = (a.n + GEMM_BM - 1) / GEMM_BM;
+    sh.nt = (a.w.rows + GEMM_BN - 1) / GEMM_BN;
+    // one slice of vector tiles per XCD (at 2048 vectors: 256 KiB of operand
+    // per 32-vector tile, eight per XCD) unless there are fewer vector tiles
+    sh.ga = 8;
+    while (sh.ga > 1 && sh.ga > sh.mt) sh.ga >>= 1;
+    sh.mts = (sh.mt + sh.ga - 1) / sh.ga;
+    sh.nts = (sh.nt + 8 / sh.ga - 1) / (8 / sh.ga);
+    const long wgs = 8L * sh.mts * sh.nts;
+    if (wgs > 0x7fffffffL) return -6;
+    // fewer than four work-groups per CU (the grids that two ranges of twice
+    // the work would also serve): each range is summed in two halves, so a
+    // range costs no precision against two of half its length (2048 inputs:
+    // 1.39e-7 of the result in 2-norm, 1.69e-7 in one chain; 20.2 us against
+    // 19.7 at 2048 x 2048 x 512 vectors).  The 16 KiB of LDS it takes would
+    // cost fuller grids a fourth work-group per CU.
+    sh.fq = (long)sh.mt * sh.nt * ks < 4L * gemv_cus() ? 2 * ((sh.kq + 3) / 4) : 0;
+    const size_t lds = (size_t)GEMM_STAGES * 4 * 4 * 2 * GEMM_BM * 16 + (sh.fq ? (size_t)GEMM_NT * 64 : 0);
+    const dim3 grid((unsigned)wgs, (unsigned)ks), block(GEMM_NT);
+    if (a.ev_start)
+        hipExtLaunchKernelGGL((k_gemm<DT>), grid, block, lds, s, a.ev_start, ks > 1 ? nullptr : a.ev_stop, 0, a, sh);
+    else
+        hipLaunchKernelGGL((k_gemm<DT>), grid, block, lds, s, a, sh);
+    return ks > 1 ? launch_gemm_finish(a, epi, ks, s) : 0;
 }

@@ -34,6 +34,9 @@ int launch_gemv_q6k(const GemvArgs &a, int epi, hipStream_t s);
 int launch_gemm_q4k(const GemvArgs &a, int epi, hipStream_t s);
 int launch_gemm_q6k(const GemvArgs &a, int epi, hipStream_t s);
 
+// four floats at any float address
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
 size_t act_bytes(int K, int n)
 {
     const size_t blocks = (size_t)((K / 32 + 3) / 4) * 4;
@@ -76,6 +79,14 @@ int launch_gemm(const GemvArgs &a, int epi, hipStream_t s)
 size_t gemm_part_floats(const QTensor &w, int n)
 {
     const int ks = gemm_ks(w, n, (size_t)-1);
+    return ks > 1 ? (size_t)ks * n * w.rows : 0;
+}
+
+size_t gemm_part_least(const QTensor &w, int n)
+{
+    const long tiles = (long)((n + 63) / 64) * ((w.rows + 127) / 128);
+    int ks = 1;
+    while (ks < 4 && tiles * ks < 2L * gemv_cus() && w.fold * w.block_quads / (2 * ks) >= 8) ks *= 2;
     return ks > 1 ? (size_t)ks * n * w.rows : 0;
 }
 
@@ -193,6 +204,81 @@ int launch_gemv_b_finish(const GemvArgs &a, int epi, int splits, int ss_count, h
     return 0;
 }
 
+// k-split finish of the prompt GEMM: a work-group per 16 vectors and BR rows
+// (a piece of eight inputs or four rows per thread, see epi_runs), the
+// partial sums read 16 bytes at a time, up to four ranges in flight.
+template <int EPI> constexpr int gfin_rows() { return EPI == EPI_SWIGLU ? 256 : EPI == EPI_RESID ? 128 : 64; }
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_gemm_finish(GemvArgs a, int ks)
+{
+#pragma clang fp contract(off)
+    constexpr int BR = gfin_rows<EPI>();
+    __shared__ float s_nrm[16];
+    const int m0 = blockIdx.y * 16, r0 = blockIdx.x * BR, tid = threadIdx.x;
+    const size_t kstride = (size_t)a.n * a.w.rows;
+    if (a.in.ss) {
+        gemm_norms<16, 256>(a, m0, s_nrm, tid);
+        __syncthreads();
+    }
+    // rows r0 + rl .. +3 of vector m0 + vi (callers ask for real ones only;
+    // the last of an odd row count re-read its own row)
+    auto src = [&](int vi, int rl) {
+        const int left = a.w.rows - (r0 + rl);
+        const float *p = a.part + (size_t)(m0 + vi) * a.w.rows + r0 + rl;
+        f32x4 y = {};
+        for (int k = 0; k < ks; k += 4) {
+            f32x4 q[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const float *pk = p + (size_t)min(k + u, ks - 1) * kstride;
+                if (left >= 4) {
+                    const f4u t = *(const f4u *)pk;
+                    q[u] = f32x4{t[0], t[1], t[2], t[3]};
+                } else {
+                    q[u] = f32x4{pk[0], pk[min(1, left - 1)], pk[min(2, left - 1)], 0.0f};
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (k + u < ks) y += q[u];
+        }
+        if (a.in.ss) y *= s_nrm[vi];
+        return y;
+    };
+    if constexpr (EPI == EPI_STORE) {
+        const int vi = tid >> 4, rl = 4 * (tid & 15), left = a.w.rows - (r0 + rl);
+        if (m0 + vi >= a.n || left <= 0) return;
+        const f32x4 y = src(vi, rl);
+        float *o = a.out + (size_t)(m0 + vi) * a.out_stride + r0 + rl;
+        if (left >= 4) *(f4u *)o = f4u{y[0], y[1], y[2], y[3]};
+        else
+            for (int i = 0; i < left; i++) o[i] = y[i];
+    } else {
+        epi_runs<EPI, 16, BR, 256>(a, src, m0, r0, tid);
+    }
+}
+
+template <int EPI>
+static void launch_gfin(const GemvArgs &a, int ks, hipStream_t s)
+{
+    constexpr int BR = gfin_rows<EPI>();
+    const dim3 grid((a.w.rows + BR - 1) / BR, (a.n + 15) / 16), block(256);
+    if (a.ev_stop) hipExtLaunchKernelGGL(k_gemm_finish<EPI>, grid, block, 0, s, nullptr, a.ev_stop, 0, a, ks);
+    else hipLaunchKernelGGL(k_gemm_finish<EPI>, grid, block, 0, s, a, ks);
+}
+
+int launch_gemm_finish(const GemvArgs &a, int epi, int ks, hipStream_t s)
+{
+    switch (epi) {
+    case EPI_STORE: launch_gfin<EPI_STORE>(a, ks, s); break;
+    case EPI_RESID: launch_gfin<EPI_RESID>(a, ks, s); break;
+    case EPI_SWIGLU: launch_gfin<EPI_SWIGLU>(a, ks, s); break;
+    default: launch_gfin<EPI_QKV>(a, ks, s); break;
+    }
+    return 0;
+}
+
 // Standalone operand preparation: one thread per (vector, block of 32,
 // k-group), i.e. per 16-byte piece of the operand's high and low rows: two
 // 4-float loads, two 16-byte stores; the block's sum of squares meets over
@@ -206,8 +292,6 @@ int launch_gemv_b_finish(const GemvArgs &a, int epi, int splits, int ss_count, h
 // vectors of one block (512 contiguous bytes stored per k-group, whole
 // 128-byte lines read); with fewer, one vector of 16 blocks.
 // x and norm_w carry no alignment beyond a float's.
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-
 template <int VS>
 __global__ __launch_bounds__(256) void k_act_prep(const float *__restrict__ x, int x_stride, int K, int n, ActOut o)
 {

@@ -253,8 +253,8 @@ int launch_gemv(const GemvArgs &a, int epi, hipStream_t s);
 // partial sums (0 when it does not split k).
 size_t gemv_part_floats(const QTensor &w, int n);
 // Most k ranges a split-K prompt GEMM takes (its partial sums go to a.part).
-#define GEMM_KS_MAX 4
-// The same product for many vectors (prompt tokens): 64-vector x 128-row
+#define GEMM_KS_MAX 16
+// The same product for many vectors (prompt tokens): 32-vector x 128-row
 // output tiles, epilogues EPI_STORE..EPI_QKV; any n >= 1.  With a.part,
 // narrow matrices whose tiles would not fill the chip split k (fp32 partial
 // sums, then the k-split finish).
@@ -262,6 +262,11 @@ int launch_gemm(const GemvArgs &a, int epi, hipStream_t s);
 // Partial-sum floats the split-K prompt GEMM of n vectors over w takes when
 // given room without limit (0 when it does not split).
 size_t gemm_part_floats(const QTensor &w, int n);
+// Of these, what a call on a caller's arena or the fixed scratch insists on
+// (a part_cap between the two splits into fewer ranges): up to four ranges of
+// eight block quads or more, where 64-vector tiles would not fill the chip
+// twice.  It sets which calls a given amount of scratch takes, and stays.
+size_t gemm_part_least(const QTensor &w, int n);
 // x [n][x_stride] fp32 -> operand (and sum-of-squares partials per 32 inputs).
 int launch_act_prep(const float *x, int x_stride, int K, int n, const ActOut &o, hipStream_t s);
 // Operand bytes for K inputs (padded to whole block quads) and n vectors.

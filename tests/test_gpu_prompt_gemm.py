@@ -6,6 +6,7 @@ import pytest
 import libcmol_amd.native as native
 from libcmol_amd import synth
 from oracle import oracle as O
+from tests.qdata import random_blocks
 
 pytestmark = pytest.mark.gpu
 ATOL, RTOL = 1e-4, 1e-3
@@ -40,3 +41,49 @@ def test_prompt_epilogues_match_oracle(gpu, model_dir, wtype, heads, kv, d_model
             assert np.all(np.abs(got - ref) <= ATOL + RTOL * np.abs(ref))
     m.close()
     om.close()
+
+
+def check_gemm(ctx, dtype, rows, cols, fold, n, norm):
+    raw = random_blocks(dtype, rows, cols, seed=rows + 3 * cols + n)
+    rng = np.random.default_rng(n + rows)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    w = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32) if norm else None
+    t = ctx.qtensor([raw], dtype, cols, [rows], fold=fold)
+    got = ctx.gemm(t, x, w)
+    if norm:
+        x64 = x.astype(np.float64)
+        x = (x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-5) * w).astype(np.float32)
+    want = O.matmul(raw, np.ascontiguousarray(x.T), rows, cols, dtype, O.AVX512).T
+    # Both sides sum thousands of terms in fp32, in their own orders: rounding
+    # of each partial sum (2^-24 of it, the sums growing to the outputs' rms
+    # over up to 512 blocks) adds up to 2..5e-7 of the rms per output, whatever
+    # the output's own size; the largest of some thousands stays below 10 sigma
+    tol = ATOL + RTOL * np.abs(want) + 5e-6 * np.sqrt(np.mean(want.astype(np.float64) ** 2))
+    assert np.all(np.abs(got - want) <= tol), f"{dtype} {rows}x{cols} fold {fold} n {n}"
+
+
+# k ranges 1 (one quad pair), 2, 4, 8 and 16, the last range short or empty
+# (20 quads in 8 ranges of 3), ranges summed in one chain and in two halves,
+# folded tensors, and row counts that are no multiple of 4 with partial sums
+@pytest.mark.parametrize("dtype", [2, 8, 12])
+@pytest.mark.parametrize("rows,cols,fold,n,norm", [
+    (128, 256, 1, 33, True), (130, 512, 1, 40, False), (131, 1024, 1, 33, True), (257, 2560, 1, 64, True),
+    (129, 8192, 1, 35, False), (96, 16384, 1, 33, True), (512, 2048, 2, 65, True), (512, 2048, 4, 100, False),
+    (4096, 512, 1, 1056, False), (4096, 512, 1, 1024, True)])
+def test_gemm_k_ranges_match_oracle(gpu, dtype, rows, cols, fold, n, norm):
+    ctx = gpu.Ctx(512 << 20)
+    check_gemm(ctx, dtype, rows, cols, fold, n, norm)
+    ctx.close()
+
+
+def test_gemm_small_arena_takes_fewer_ranges(gpu):
+    """An arena with room for fewer k ranges' partial sums than the product
+    would take: the call still runs, on fewer ranges."""
+    rows, cols, n = 256, 4096, 64
+    sizes = [gpu.lib().cmolhip_qtensor_bytes(2, rows, cols, 1), rows * cols // 32 * 18, n * cols * 4, n * rows * 4,
+             gpu.lib().cmolhip_act_bytes(cols, n)]
+    # 32 quads on two 128-row tiles x two 32-vector tiles: 16 ranges of two,
+    # 1 MiB of partial sums; the arena has room for four, 256 KiB
+    ctx = gpu.Ctx(sum(sizes) + 4 * n * rows * 4 + 4096)
+    check_gemm(ctx, 2, rows, cols, 1, n, False)
+    ctx.close()
