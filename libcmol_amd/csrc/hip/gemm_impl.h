@@ -131,30 +131,6 @@ __device__ __forceinline__ void gemm_norms(const GemvArgs &a, int m0, float *s_n
     if (sub == 0) s_nrm[vi] = 1.0f / sqrtf(s / (float)a.w.cols + a.in.eps);
 }
 
-// Operand piece (block b, k-group g) of vector v from its eight inputs in
-// natural order (the first four, then the second four: see piece_k): the
-// high and low rows' 16 bytes each.
-__device__ __forceinline__ void act_put8(const ActOut &o, int v, int b, int g, int k0, int k1, const f32x4 &x0,
-                                         const f32x4 &x1)
-{
-#pragma clang fp contract(off)
-    f16x8 hi, lo;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const float x = e < 4 ? x0[e] : x1[e - 4];
-        const float t = (o.norm_w ? o.norm_w[(e < 4 ? k0 : k1 - 4) + e] * x : x) * ACT_SCALE;
-        hi[e] = (_Float16)t;
-        lo[e] = (_Float16)((t - (float)hi[e]) * LO_SCALE);
-    }
-    if (o.dt != DT_Q8_0) {
-        hi = __builtin_shufflevector(hi, hi, 0, 2, 1, 3, 4, 6, 5, 7);
-        lo = __builtin_shufflevector(lo, lo, 0, 2, 1, 3, 4, 6, 5, 7);
-    }
-    f16x8 *dst = (f16x8 *)(o.q + (((size_t)b * 4 + g) * o.nrows + 2 * v) * 8);
-    dst[0] = hi;
-    dst[1] = lo;
-}
-
 // Epilogues of a tile of BM vectors x BR output rows (vectors m0 .., rows
 // r0 .., r0 a multiple of BR) by NT threads; src(vi, rl) gives the products of
 // vector m0 + vi and rows r0 + rl .. +3, scaled.  EPI_RESID and EPI_SWIGLU:

@@ -312,9 +312,8 @@ int launch_attn_merge_wave(const AttnArgs &a, hipStream_t s);
 // seqlen.  kv_hl (fp32 caches only): attn_prompt_kv_bytes of scratch for the
 // high/low f16 copy of the session's cache positions 0 .. last-1.
 int launch_attn_prompt(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s);
+// (attn_prompt.hip)
 size_t attn_prompt_kv_bytes(int n_kv, int d_head, int max_ctx);
-// Its fp16-cache kernel and split merge.
-int launch_attn_prompt16(const AttnArgs &a, hipStream_t s);
 
 // QK-norm models (src/attn.c:62-101): the QKV matvec stores raw q|k|v rows;
 // this stage normalises each q and k head (RMSNorm over d_head, weights
@@ -491,4 +490,56 @@ __device__ inline void act_put(const ActOut &o, int n, int k, float v)
     const size_t base = (((size_t)b * 4 + g) * o.nrows + 2 * n) * 8 + e;
     M::st(o.q + base, hi);
     M::st(o.q + base + 8, lo);
+}
+
+// Operand piece (block b, k-group g) of vector v from its eight inputs, x0
+// inputs k0 .. +3 and x1 inputs k1 .. +3 (k1 = k0 + 4 for Q8_0 consumers, else
+// k0 + 16): the high and low rows' 16 bytes each.
+__device__ __forceinline__ void act_put8(const ActOut &o, int v, int b, int g, int k0, int k1, const f32x4 &x0,
+                                         const f32x4 &x1)
+{
+#pragma clang fp contract(off)
+    f16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float x = e < 4 ? x0[e] : x1[e - 4];
+        const float t = (o.norm_w ? o.norm_w[(e < 4 ? k0 : k1 - 4) + e] * x : x) * ACT_SCALE;
+        hi[e] = (_Float16)t;
+        lo[e] = (_Float16)((t - (float)hi[e]) * LO_SCALE);
+    }
+    if (o.dt != DT_Q8_0) {
+        hi = __builtin_shufflevector(hi, hi, 0, 2, 1, 3, 4, 6, 5, 7);
+        lo = __builtin_shufflevector(lo, lo, 0, 2, 1, 3, 4, 6, 5, 7);
+    }
+    f16x8 *dst = (f16x8 *)(o.q + (((size_t)b * 4 + g) * o.nrows + 2 * v) * 8);
+    dst[0] = hi;
+    dst[1] = lo;
+}
+
+// Inputs k .. k+3 (k a multiple of 4) of vector v: eight bytes of the high
+// and of the low row.
+__device__ __forceinline__ void act_put4(const ActOut &o, int v, int k, const f32x4 &x)
+{
+#pragma clang fp contract(off)
+    f16x4 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float t = (o.norm_w ? o.norm_w[k + e] * x[e] : x[e]) * ACT_SCALE;
+        hi[e] = (_Float16)t;
+        lo[e] = (_Float16)((t - (float)hi[e]) * LO_SCALE);
+    }
+    const int b = k >> 5, kk = k & 31;
+    int g, e0;
+    if (o.dt == DT_Q8_0) {
+        g = kk >> 3;
+        e0 = kk & 4;
+    } else {
+        hi = __builtin_shufflevector(hi, hi, 0, 2, 1, 3);
+        lo = __builtin_shufflevector(lo, lo, 0, 2, 1, 3);
+        g = (kk & 15) >> 2;
+        e0 = kk >> 4 << 2;
+    }
+    _Float16 *dst = o.q + (((size_t)b * 4 + g) * o.nrows + 2 * v) * 8 + e0;
+    *(f16x4 *)dst = hi;
+    *(f16x4 *)(dst + 8) = lo;
 }

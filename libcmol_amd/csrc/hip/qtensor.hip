@@ -268,7 +268,7 @@ __global__ __launch_bounds__(256) void k_embed(QTensor t, const int32_t *__restr
     const int tok = token[s * token_stride];
     if (argmax && blockIdx.x == 0)
         for (int i = threadIdx.x; i < ARGMAX_SLOTS; i += blockDim.x) argmax[(size_t)s * ARGMAX_SLOTS + i] = 0ull;
-    embed_group<DT, StPlain>(t, tok, blockIdx.x * blockDim.x + threadIdx.x, x + (size_t)s * x_stride, o, s);
+    embed_group<DT>(t, tok, blockIdx.x * blockDim.x + threadIdx.x, x + (size_t)s * x_stride, o, s);
 }
 
 int launch_embed(const QTensor &t, const int32_t *token, int token_stride, float *x,

@@ -81,7 +81,7 @@ __device__ void block_values_g(const QTensor &t, int row, int b, int g, float *d
 // read row 0): x[32b + k] = value, the consumer operand of vector s, and the
 // per-block sum of squares (the 4 threads of a block are consecutive lanes).
 // Every lane of the wave must call it (shuffles).
-template <int DT, typename M>
+template <int DT>
 __device__ inline void embed_group(const QTensor &t, int tok, int gid, float *x, const ActOut &o, int s)
 {
 #pragma clang fp contract(off)
@@ -92,15 +92,24 @@ __device__ inline void embed_group(const QTensor &t, int tok, int gid, float *x,
     if (b < nb) {
         float val[8];
         block_vals8<DT>(t, tok, b, g, val);
-        for (int e = 0; e < 8; e++) {
-            const int k = 32 * b + kmap(DT, g, e);
-            if (x) M::st(x + k, val[e]);
-            ss += val[e] * val[e];
-            if (o.q) act_put<M>(o, s, k, val[e]);
+        // the lane group's inputs in natural order, 32b + o0 .. +3 and o1 .. +3
+        // (the nibble decoders give each four as 0, 2, 1, 3)
+        constexpr bool Q8 = DT == DT_Q8_0;
+        const int o0 = Q8 ? 8 * g : 4 * g, o1 = Q8 ? o0 + 4 : o0 + 16;
+        const f32x4 v0 = {val[0], val[Q8 ? 1 : 2], val[Q8 ? 2 : 1], val[3]};
+        const f32x4 v1 = {val[4], val[Q8 ? 5 : 6], val[Q8 ? 6 : 5], val[7]};
+        for (int e = 0; e < 8; e++) ss += val[e] * val[e];
+        if (x) {
+            *(f32x4 *)(x + 32 * b + o0) = v0;
+            *(f32x4 *)(x + 32 * b + o1) = v1;
+        }
+        if (o.q) {
+            act_put4(o, s, 32 * b + o0, v0);
+            act_put4(o, s, 32 * b + o1, v1);
         }
     }
     // per-block sum over the 4 lane groups (lanes 4b..4b+3 of the wave)
     ss += __shfl_xor(ss, 1, 64);
     ss += __shfl_xor(ss, 2, 64);
-    if (b < nb && g == 0 && o.ss) M::st(o.ss + (size_t)s * o.ss_stride + b, ss);
+    if (b < nb && g == 0 && o.ss) o.ss[(size_t)s * o.ss_stride + b] = ss;
 }
