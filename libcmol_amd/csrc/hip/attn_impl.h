@@ -689,6 +689,198 @@ __device__ __forceinline__ void attn_piece_mfw(const AttnArgs &a, int kvh, int n
     __syncthreads();   // the LDS areas may be reused by the caller
 }
 
+// The same piece over an fp32 cache with at most four query heads per kv
+// head (d_head 64 / 128), on the vector ALUs; the four waves independent as
+// in attn_piece_mfw, no barrier inside the walk:
+//   * scores: four lanes per position, each a quarter of the K row
+//     (interleaved 16-byte pieces, loaded straight into registers one step
+//     ahead) against the same pieces of the query heads from LDS (broadcast
+//     reads); the four partial dots meet in two quad_perm steps and lane j
+//     keeps head j's score, so 64 lanes hold 16 positions x 4 heads;
+//   * lazy online softmax as in attn_piece_mfw, per head j over the lanes
+//     l % 4 = j; the 64 weights go to the wave's LDS row;
+//   * weighted sum: lanes along the V row (16 bytes each, 1024 / d_head / 4
+//     rows per load), each row's four weights read as one broadcast 16-byte
+//     LDS read.
+// Same partial format as attn_split; all arithmetic fp32.
+// Bound by the K/V bytes once there are rounds of pieces: 32 contexts of
+// 512..4096 positions at 16/4 heads of 128, 227 MB, 41.4 us (5.5 TB/s) where
+// the split grid (attn.hip, k_attn_h: a 64-position split per 512-thread
+// work-group, one per CU by its LDS) took 85.5; 8 contexts of 64..4096 22.2 ->
+// 13.2 us.
+template <int DH, typename M>
+__device__ __forceinline__ void attn_piece_fw(const AttnArgs &a, int kvh, int n, int t0, int cnt, bool single,
+                                              size_t sbase, size_t kvo)
+{
+#pragma clang fp contract(off)
+    constexpr int NT = 256, NW = NT / 64, HM = 4;
+    constexpr int KP = DH / 16;      // 16-byte K pieces per lane
+    constexpr int LR = DH / 4;       // lanes per V row
+    constexpr int RPI = 64 / LR;     // V rows per load
+    constexpr int VI = 16 / RPI;     // V loads per step
+    const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int pos = lane >> 2, j = lane & 3, vr = lane / LR, dq = lane % LR;
+    const int G = a.n_heads / a.n_kv;
+    cnt = __builtin_amdgcn_readfirstlane(cnt);   // the same in every lane
+    t0 = __builtin_amdgcn_readfirstlane(t0);
+    const int nst = (cnt + 63) / 64;
+
+    __shared__ __attribute__((aligned(16))) float qs[HM][DH];
+    __shared__ __attribute__((aligned(16))) float wsm[NW][64];
+    __shared__ __attribute__((aligned(16))) float xo[NW][HM][DH];
+    __shared__ float xm[NW][HM], xl[NW][HM];
+
+    const size_t off = kvo + (size_t)kvh * a.max_ctx * DH + (size_t)t0 * DH;   // kvo: the vector's cache base
+    const char *kb = (const char *)uniform_ptr((const float *)a.kv.k_base + off);
+    const char *vb = (const char *)uniform_ptr((const float *)a.kv.v_base + off);
+    f32x4 kr[KP], vv[VI];
+    auto load_k = [&](int st) {
+        const unsigned p = (unsigned)min(64 * st + 16 * wid + pos, cnt - 1);
+#pragma unroll
+        for (int i = 0; i < KP; i++) kr[i] = ldg((const f32x4 *)(kb + 4u * (p * DH + 4 * (j + 4 * i))));
+    };
+    auto load_v = [&](int st) {
+#pragma unroll
+        for (int i = 0; i < VI; i++) {
+            const unsigned p = (unsigned)min(64 * st + 16 * wid + i * RPI + vr, cnt - 1);
+            vv[i] = ldg((const f32x4 *)(vb + 4u * (p * DH + 4 * dq)));
+        }
+    };
+    const float *qn = a.q + (size_t)n * a.q_stride + (size_t)kvh * G * DH;
+    float qv[HM * DH / NT];
+#pragma unroll
+    for (int i = 0; i < HM * DH / NT; i++) {
+        const int e = tid + i * NT;
+        qv[i] = e < G * DH ? ldg(qn + e) : 0.0f;
+    }
+    load_k(0);
+    load_v(0);
+#pragma unroll
+    for (int i = 0; i < HM * DH / NT; i++) (&qs[0][0])[tid + i * NT] = qv[i];
+    __syncthreads();
+
+    const float scale = 1.0f / sqrtf((float)DH);
+    constexpr float L2E = 1.44269504088896341f;   // log2(e)
+    const float c2 = scale * L2E, lazy = ATT_LAZY_T / scale;
+    f32x4 o[HM];
+#pragma unroll
+    for (int h = 0; h < HM; h++) o[h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // head j of this lane: reference maximum (raw units), -m c2 and the
+    // lane's sum of weights
+    float m = -INFINITY, mk = 0.0f, lsum = 0.0f;
+
+    for (int st = 0; st < nst; st++) {
+        const int pb = 64 * st + 16 * wid;   // the wave's first position of the step
+        if (pb >= cnt) break;                // every later row of the wave is past the piece too
+        // the query is read from LDS in every step, one piece ahead of its use;
+        // z (zero) depends on the sums so far, or the compiler would gather
+        // the step's reads, 128 registers of them, at the top
+        int z = 0;
+        float dot[HM];
+        f32x4 q4[2][HM];
+#pragma unroll
+        for (int h = 0; h < HM; h++) {
+            dot[h] = 0.0f;
+            q4[0][h] = *(const f32x4 *)&qs[h][4 * j];
+        }
+#pragma unroll
+        for (int i = 0; i < KP; i++) {
+            asm volatile("" : "+s"(z) : "v"(dot[HM - 1]));
+            if (i + 1 < KP) {
+#pragma unroll
+                for (int h = 0; h < HM; h++) q4[(i + 1) & 1][h] = *(const f32x4 *)&qs[h][4 * (z + j) + 16 * (i + 1)];
+            }
+#pragma unroll
+            for (int h = 0; h < HM; h++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) dot[h] = fmaf(q4[i & 1][h][e], kr[i][e], dot[h]);
+        }
+        // unconditional (past the piece every lane re-reads its last row): a
+        // branch here would let the compiler sink the sums below it
+        load_k(st + 1);
+#pragma unroll
+        for (int h = 0; h < HM; h++) {
+            dot[h] += __int_as_float(
+                __builtin_amdgcn_mov_dpp(__float_as_int(dot[h]), 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+            dot[h] += __int_as_float(
+                __builtin_amdgcn_mov_dpp(__float_as_int(dot[h]), 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+        }
+        float s = j & 1 ? (j & 2 ? dot[3] : dot[1]) : (j & 2 ? dot[2] : dot[0]);
+        s = pb + pos < cnt ? s : -INFINITY;
+        if (__ballot(s > m + lazy)) {
+            float cm = s;
+#pragma unroll
+            for (int x = 4; x < 64; x <<= 1) cm = fmaxf(cm, __shfl_xor(cm, x, 64));
+            const float mn = fmaxf(m, cm);
+            const float mref = mn == -INFINITY ? 0.0f : mn;
+            const float al = mn == m ? 1.0f : __builtin_amdgcn_exp2f((m - mref) * c2);
+            m = mn;
+            mk = -mref * c2;
+            lsum *= al;
+#pragma unroll
+            for (int h = 0; h < HM; h++) o[h] *= __int_as_float(__builtin_amdgcn_readlane(__float_as_int(al), h));
+        }
+        const float e = __builtin_amdgcn_exp2f(fmaf(s, c2, mk));
+        lsum += e;
+        wsm[wid][lane] = e;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < VI; i++) {
+            const f32x4 w = *(const f32x4 *)&wsm[wid][4 * (i * RPI + vr)];
+#pragma unroll
+            for (int h = 0; h < HM; h++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) o[h][d] = fmaf(w[h], vv[i][d], o[h][d]);
+        }
+        __builtin_amdgcn_wave_barrier();
+        load_v(st + 1);
+    }
+
+    // the wave's sums over its lanes, then the waves per head
+#pragma unroll
+    for (int x = 4; x < 64; x <<= 1) lsum += __shfl_xor(lsum, x, 64);
+#pragma unroll
+    for (int h = 0; h < HM; h++)
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+#pragma unroll
+            for (int x = LR; x < 64; x <<= 1) o[h][d] += __shfl_xor(o[h][d], x, 64);
+    if (pos == 0) {
+        xm[wid][j] = m * scale;   // natural units, as the partials carry it
+        xl[wid][j] = lsum;
+    }
+    if (vr == 0) {
+#pragma unroll
+        for (int h = 0; h < HM; h++) *(f32x4 *)&xo[wid][h][4 * dq] = o[h];
+    }
+    __syncthreads();
+    for (int i = tid; i < G * DH; i += NT) {
+        const int h = i / DH, d = i % DH;
+        float mx = xm[0][h];
+#pragma unroll
+        for (int w = 1; w < NW; w++) mx = fmaxf(mx, xm[w][h]);
+        float lt = 0.0f, ot = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const float f = xm[w][h] > -INFINITY ? expf(xm[w][h] - mx) : 0.0f;
+            lt += xl[w][h] * f;
+            ot += xo[w][h][d] * f;
+        }
+        if (single) {
+            const float fv = ot / lt;
+            const int kk = (kvh * G + h) * DH + d;
+            if (a.out) M::st(a.out + (size_t)n * a.out_stride + kk, fv);
+            if (a.next.q) act_put<M>(a.next, n, kk, fv);
+        } else {
+            M::st(a.po + (sbase + h) * DH + d, ot);
+            if (d == 0) {
+                M::st(a.pm + sbase + h, mx);
+                M::st(a.pl + sbase + h, lt);
+            }
+        }
+    }
+}
+
 // One split of attn_split's grid: positions sp*split .. of vector n; a
 // session that fits one split is finished here.
 template <int DH, typename M>
@@ -706,12 +898,13 @@ __device__ __forceinline__ void attn_split_mf(const AttnArgs &a, int kvh, int sp
 // laid end to end on one line, each preceded by ATT_BAL_PAD positions that
 // stand for the fixed cost of starting a piece (query load, pipeline fill);
 // range w of a kv head is the line's [wR, wR + R) with
-// R = max(split, ceil(line / B)), so the ranges hold about the same number
+// R = max(split, ceil(line / B)) (fp32: at least 128), so the ranges hold about the same number
 // of cached rows whatever the mix of lengths.  The cut of vector n's
 // positions that falls in range w is a piece; pieces are in line order, so
 // slot w + n is unique to it, and vector n's pieces are the consecutive
 // slots w0 + n .. w1 + n.  Work-group k of a kv head (k < B + n_vectors)
-// runs the piece of slot k, if any, with attn_piece_mfw: the whole context
+// runs the piece of slot k, if any, with attn_piece_mfw (fp16 cache) or
+// attn_piece_fw (fp32): the whole context
 // is finished here, a cut one written as the partial [kvh][k][G] that
 // k_attn_merge combines.
 // Unlike the split grid, no work-group starts only to find its split past
@@ -746,11 +939,14 @@ __device__ __forceinline__ int attn_bal_range(const AttnArgs &a, int l0)
     int t = lane < a.n ? l0 + ATT_BAL_PAD : 0;
     for (int b = 64; b < a.n; b += 64) t += b + lane < a.n ? attn_len(a, b + lane) + ATT_BAL_PAD : 0;
     const int line = wave_sum_i(t);
-    return max(a.split, (line + a.bal - 1) / a.bal);
+    // fp32: two steps of the work-group at least, or starting and merging the
+    // pieces outweighs them (16/4 heads of 128, 8 contexts of 64..4096: ranges
+    // of 64 positions 15.2 + 5.7 us, of 128 13.2 + 4.6)
+    return max(a.kv_f16 ? a.split : max(a.split, 128), (line + a.bal - 1) / a.bal);
 }
 
-template <int DH, typename M>
-__device__ __forceinline__ void attn_bal_mf(const AttnArgs &a, int kvh, int k)
+template <int DH, typename KT, typename M>
+__device__ __forceinline__ void attn_bal_run(const AttnArgs &a, int kvh, int k)
 {
     const int lane = threadIdx.x & 63;
     const int G = a.n_heads / a.n_kv;
@@ -763,7 +959,7 @@ __device__ __forceinline__ void attn_bal_mf(const AttnArgs &a, int kvh, int k)
     int base = 0, s = -1, pj = 0, lj = 0, sj = 0;
     for (int b = 0; b < a.n; b += 64) {
         const int L = b == 0 ? l0 : attn_len(a, b + lane);
-        const int slot = a.kv.slot_ids && b + lane < a.n ? a.kv.slot_ids[b + lane] : 0;
+        const int slot = b + lane >= a.n ? 0 : a.kv.slot_ids ? a.kv.slot_ids[b + lane] : b + lane;
         const int v = b + lane < a.n ? L + ATT_BAL_PAD : 0;
         const int inc = wave_scan_i(v);
         const int p0 = base + inc - v + ATT_BAL_PAD;   // line offset of the vector's position 0
@@ -782,8 +978,11 @@ __device__ __forceinline__ void attn_bal_mf(const AttnArgs &a, int kvh, int k)
     if (s < 0) return;   // no piece in this slot
     const int w = k - s;
     const int r0 = max(w * R - pj, 0), r1 = min((w + 1) * R - pj, lj);
-    const size_t kvo = (a.kv.slot_ids ? (size_t)sj * a.kv.slot_stride : 0) + a.kv.layer_off;
-    attn_piece_mfw<DH, M>(a, kvh, s, r0, r1 - r0, r0 == 0 && r1 == lj, ((size_t)kvh * (a.bal + a.n) + k) * G, kvo);
+    const size_t kvo = (size_t)sj * a.kv.slot_stride + a.kv.layer_off;
+    const bool single = r0 == 0 && r1 == lj;
+    const size_t sbase = ((size_t)kvh * (a.bal + a.n) + k) * G;
+    if constexpr (sizeof(KT) == 2) attn_piece_mfw<DH, M>(a, kvh, s, r0, r1 - r0, single, sbase, kvo);
+    else attn_piece_fw<DH, M>(a, kvh, s, r0, r1 - r0, single, sbase, kvo);
 }
 
 // Merge of the splits of one (query head, vector) by NT threads:

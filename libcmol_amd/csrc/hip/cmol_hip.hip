@@ -514,12 +514,9 @@ int cmolhip_attn_decode(cmolhip_ctx_t *c, int n, const float *q, const void *kca
     int rc = E_OK;
     do {
         float *pm, *pl, *po;
-        int32_t *ids;
         const size_t np = (size_t)n * n_kv * ms * G;
-        if ((rc = arena_get(c, np, &pm)) || (rc = arena_get(c, np, &pl)) ||
-            (rc = arena_get(c, np * d_head, &po)) || (rc = arena_get(c, (size_t)n, &ids)))
+        if ((rc = arena_get(c, np, &pm)) || (rc = arena_get(c, np, &pl)) || (rc = arena_get(c, np * d_head, &po)))
             break;
-        if ((rc = launch_iota(ids, n, c->stream))) break;   // cache i belongs to session i
         AttnArgs a{};
         a.q = q;
         a.q_stride = n_heads * d_head;
@@ -527,7 +524,7 @@ int cmolhip_attn_decode(cmolhip_ctx_t *c, int n, const float *q, const void *kca
         a.kv.v_base = (void *)vcache;
         a.kv.slot_stride = (size_t)n_kv * max_ctx * d_head;
         a.kv.layer_off = 0;
-        a.kv.slot_ids = ids;
+        a.kv.slot_ids = nullptr;   // cache i belongs to session i
         a.seqlen = seqlen;
         a.seqlen_stride = 1;
         a.n = n;
@@ -538,7 +535,7 @@ int cmolhip_attn_decode(cmolhip_ctx_t *c, int n, const float *q, const void *kca
         a.kv_f16 = kv_f16;
         a.split = split;
         a.max_splits = ms;
-        a.bal = attn_bal_wgs(n, n_kv, d_head, kv_f16, ms);
+        a.bal = attn_bal_wgs(n, n_heads, n_kv, d_head, kv_f16, ms);
         a.pm = pm;
         a.pl = pl;
         a.po = po;
@@ -1254,7 +1251,7 @@ int enqueue_step(cmolhip_model *m, Batch &B, int n, hipStream_t st)
         at.kv_f16 = hp.kv_f16;
         at.split = m->split;
         at.max_splits = m->max_splits;
-        at.bal = attn_bal_wgs(n, hp.n_kv_heads, hp.d_head, hp.kv_f16, m->max_splits);
+        at.bal = attn_bal_wgs(n, hp.n_heads, hp.n_kv_heads, hp.d_head, hp.kv_f16, m->max_splits);
         at.pm = B.pm;
         at.pl = B.pl;
         at.po = B.po;

@@ -115,8 +115,8 @@ __device__ __forceinline__ void mfma_block(f32x4 &acc, const f16x8 &xv, const f1
 
 // KV caches of one layer for a batch of activation vectors: vector n uses
 // slot slot_ids[n], whose K cache starts at k_base + slot*slot_stride +
-// layer_off elements (fp32 or fp16 per kv_f16); without slot_ids every
-// vector uses k_base + layer_off.
+// layer_off elements (fp32 or fp16 per kv_f16); without slot_ids (decode
+// attention calls) vector n uses slot n.
 struct KVRef {
     void *k_base, *v_base;
     size_t slot_stride, layer_off;
@@ -125,7 +125,7 @@ struct KVRef {
 
 __device__ inline size_t kv_offset(const KVRef &r, int n)
 {
-    return (r.slot_ids ? (size_t)r.slot_ids[n] * r.slot_stride : 0) + r.layer_off;
+    return (size_t)(r.slot_ids ? r.slot_ids[n] : n) * r.slot_stride + r.layer_off;
 }
 
 // ---------------------------------------------------------------------------
@@ -285,7 +285,7 @@ struct AttnArgs {
     int n, n_heads, n_kv, d_head, max_ctx, kv_f16;
     int split;              // positions per work-group
     int max_splits;
-    int bal;                // > 0 (fp16 cache, d_head 64..256): bal balanced ranges per
+    int bal;                // > 0 (see attn_bal_wgs): bal balanced ranges per
                             // kv head instead of one work-group per split; partials
                             // [n_kv][bal + n][G]( [d_head]), bal + n <= n * max_splits
     float *pm, *pl, *po;    // partials [n][n_kv][max_splits][G]( [d_head])
@@ -297,11 +297,12 @@ struct AttnArgs {
 int launch_attn(const AttnArgs &a, hipStream_t s);
 // Balanced ranges per kv head (AttnArgs::bal) for n vectors over a cache
 // planned with max_splits splits, or 0 where they do not apply (one vector,
-// fp32 cache, d_head outside 64..256).  The grid is bal + n work-groups per
+// d_head outside 64..256, over fp32 also 256 and more than four query heads
+// per kv head).  The grid is bal + n work-groups per
 // kv head; CMOL_ATTN_BAL=<total work-groups> sets it (0: off).  The
 // default is one round of the four work-groups a CU holds.
 #define ATT_BAL_WGS_PER_CU 4
-int attn_bal_wgs(int n, int n_kv, int d_head, int kv_f16, int max_splits);
+int attn_bal_wgs(int n, int n_heads, int n_kv, int d_head, int kv_f16, int max_splits);
 int launch_attn_bal(const AttnArgs &a, hipStream_t s);   // a.bal > 0 (launch_attn calls it)
 // The split merge with one wave per (query head, vector), d_head 64 / 128:
 // prompt passes (the split layout of launch_attn).
@@ -455,8 +456,6 @@ int launch_transpose(const float *src, float *dst, int rows, int cols, hipStream
 // The kernel seam's F32 (dtype 0) and F16 (dtype 1) weight products:
 // out[m][n] = A[m][k] . x[n][k]^T in the reference AVX-512 kernel's order.
 int launch_matmul_dense(const void *a, int dtype, const float *x, float *out, int m, int k, int n, hipStream_t s);
-// out[i] = i, i < n.
-int launch_iota(int32_t *out, int n, hipStream_t s);
 int launch_kv_synth(void *kc, void *vc, int n_kv, int max_ctx, int d_head,
                     int n_tokens, int kv_f16, uint64_t seed, hipStream_t s);
 int launch_kv_convert(const void *src, float *dst, int n_kv, int max_ctx,

@@ -155,16 +155,3 @@ int launch_transpose(const float *src, float *dst, int rows, int cols, hipStream
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
-// out[i] = i for i < n.
-__global__ void k_iota(int32_t *out, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = i;
-}
-
-int launch_iota(int32_t *out, int n, hipStream_t s)
-{
-    if (n < 1) return 0;
-    hipLaunchKernelGGL(k_iota, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out, n);
-    return hipGetLastError() == hipSuccess ? 0 : -4;
-}
