@@ -349,7 +349,7 @@ static size_t product_part_floats(const cmolhip_qtensor_t &w, int n)
 }
 static size_t product_part_least(const cmolhip_qtensor_t &w, int n)
 {
-    return n <= 32 ? gemv_part_floats(to_qt(w), n) : gemm_part_least(to_qt(w), n);
+    return n <= 32 ? gemv_part_least(to_qt(w), n) : gemm_part_least(to_qt(w), n);
 }
 
 // dy[n][rows] = W . op for a prepared operand: up to 32 vectors stream the

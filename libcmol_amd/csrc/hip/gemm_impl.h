@@ -421,10 +421,12 @@ __global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) vo
     // vectors m0 + 16h + 4(l>>4) + {0, 1, 2, 3}.  Plain and partial
     // sums leave from here (64-byte runs of a vector's rows); the other
     // epilogues take the tile through LDS, 16 bytes at a time
-    const bool direct = sh.ks > 1 || sh.epi == EPI_STORE;
+    const bool logits = sh.epi == EPI_LOGITS;
+    const bool direct = sh.ks > 1 || sh.epi == EPI_STORE || logits;
     float *tile = (float *)smem;
 #pragma unroll
     for (int h = 0; h < HG; h++) {
+        unsigned long long key[4] = {};   // EPI_LOGITS: the lane's best row per vector
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             if (halves) acc[h][j] += aside[(h * NJ + j) * GEMM_NT];
@@ -440,8 +442,23 @@ __global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) vo
                 else if (v < n && row < a.w.rows) {
                     if (sh.ks > 1) a.part[((size_t)blockIdx.y * n + v) * a.w.rows + row] = y;
                     else a.out[(size_t)v * a.out_stride + row] = y;
+                    if (logits) {
+                        const unsigned long long k = argmax_key(y, (uint32_t)row);
+                        key[e] = k > key[e] ? k : key[e];
+                    }
                 }
             }
+        }
+        if (!logits) continue;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            for (int o = 8; o > 0; o >>= 1) {
+                const unsigned long long other = __shfl_xor(key[e], o, 64);
+                key[e] = other > key[e] ? other : key[e];
+            }
+            const int v = m0 + 16 * h + 4 * (l >> 4) + e;
+            if (cl == 0 && v < n)
+                atomicMax(a.argmax + (size_t)v * ARGMAX_SLOTS + ((nt_ * 4 + wid) & (ARGMAX_SLOTS - 1)), key[e]);
         }
     }
     if (direct) return;
@@ -487,13 +504,13 @@ static inline int gemm_ks(const QTensor &w, int n, size_t part_cap)
 template <int DT>
 int launch_gemm_dt(const GemvArgs &a, int epi, hipStream_t s)
 {
-    if (epi < EPI_STORE || epi > EPI_QKV) return -6;
+    if (epi < EPI_STORE || epi > EPI_LOGITS) return -6;
     // the kernel's per-lane weight offsets are 32-bit
     if ((size_t)a.w.row_tiles * a.w.block_quads * 64 * QFmt<DT>::LANE_BYTES > 0xffffffffUL) return -6;
     GemmShape sh;
     sh.epi = epi;
     const int KQ = a.w.fold * a.w.block_quads;
-    const int ks = a.part ? gemm_ks(a.w, a.n, a.part_cap) : 1;
+    const int ks = a.part && epi != EPI_LOGITS ? gemm_ks(a.w, a.n, a.part_cap) : 1;   // (the finish has no argmax)
     sh.ks = ks;
     sh.kq = (KQ + ks - 1) / ks;
     sh.mt = (a.n + GEMM_BM - 1) / GEMM_BM;

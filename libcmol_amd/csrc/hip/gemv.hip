@@ -44,9 +44,33 @@ size_t act_bytes(int K, int n)
 }
 
 
+// Whether 9 .. 32 vectors over w run the prompt GEMM, which decodes each
+// weight once for all of them, rather than the batched matvec, which decodes
+// it once per 8 or 16 vectors but has more and shorter work-groups.  us,
+// matvec / GEMM: above 16 vectors the GEMM wins once its 128-row tiles cover
+// the CUs (32 vectors Q4_0: 22016 x 2048 16.1 / 19.9, 32768 x 2048 28.8 /
+// 20.6; Q8_0 128256 x 2048 91.8 / 62.1), for 2^26 weights or more (17 vectors
+// Q8_0 8192 x 8192 26.2 / 24.5), and for the K-quants, whose decoding costs
+// more, from 2^25 (Q4_K, 20 vectors: 22016 x 2048 30.1 / 27.3; 11008 x 2048
+// 20.1 / 18.9 with the weights in the caches, but 22.0 / 22.5 with the
+// preparation and weights from HBM) or above 2^24 (Q6_K: 11008 x 2048 29.8 /
+// 23.8, 2048 x 5632 15.8 / 16.1); up to 16 vectors from two tiles per CU on (16
+// vectors Q8_0 49152 x 2048 27.9 / 29.6, 65536 x 2048 32.4 / 30.9).
+static bool batch_by_gemm(const QTensor &w, int n)
+{
+    // (folded tensors serve one session; the GEMM's weight offsets are 32-bit)
+    if (n <= 8 || w.fold != 1 || (size_t)w.row_tiles * w.block_quads * 64 * lane_bytes_of(w.dtype) > 0xffffffffUL)
+        return false;
+    const long tiles = (w.rows + GEMM_BN - 1) / GEMM_BN, weights = (long)w.rows * w.cols;
+    if (n <= 16) return tiles >= 2L * gemv_cus();
+    return tiles >= gemv_cus() || weights >= 1L << 26 || (w.dtype == DT_Q4_K && weights >= 1L << 25) ||
+           (w.dtype == DT_Q6_K && weights > 1L << 24);
+}
+
 int launch_gemv(const GemvArgs &a, int epi, hipStream_t s)
 {
     if (a.n < 1 || a.n > 32 || a.in.nrows != 2 * a.n || !a.in.q) return -6;
+    if (batch_by_gemm(a.w, a.n)) return launch_gemm(a, epi, s);
     int rc;
     switch (a.w.dtype) {
     case DT_Q4_0: rc = launch_gemv_q4(a, epi, s); break;
@@ -91,6 +115,11 @@ size_t gemm_part_least(const QTensor &w, int n)
 }
 
 size_t gemv_part_floats(const QTensor &w, int n)
+{
+    return batch_by_gemm(w, n) ? gemm_part_floats(w, n) : gemv_part_least(w, n);
+}
+
+size_t gemv_part_least(const QTensor &w, int n)
 {
     if (!gemv_batched(w, n)) return 0;
     GbShape sh;

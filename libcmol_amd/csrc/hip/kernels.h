@@ -252,10 +252,13 @@ int launch_gemv(const GemvArgs &a, int epi, hipStream_t s);
 // Scratch floats a batched (n > 8) matvec over w needs for its k-split
 // partial sums (0 when it does not split k).
 size_t gemv_part_floats(const QTensor &w, int n);
+// What a call on a caller's arena or the fixed scratch insists on (see
+// gemm_part_least): the batched matvec's own need.
+size_t gemv_part_least(const QTensor &w, int n);
 // Most k ranges a split-K prompt GEMM takes (its partial sums go to a.part).
 #define GEMM_KS_MAX 16
 // The same product for many vectors (prompt tokens): 32-vector x 128-row
-// output tiles, epilogues EPI_STORE..EPI_QKV; any n >= 1.  With a.part,
+// output tiles; any n >= 1.  With a.part,
 // narrow matrices whose tiles would not fill the chip split k (fp32 partial
 // sums, then the k-split finish).
 int launch_gemm(const GemvArgs &a, int epi, hipStream_t s);

@@ -87,3 +87,34 @@ def test_gemm_small_arena_takes_fewer_ranges(gpu):
     ctx = gpu.Ctx(sum(sizes) + 4 * n * rows * 4 + 4096)
     check_gemm(ctx, 2, rows, cols, 1, n, False)
     ctx.close()
+
+
+# batches of 9..32 that the tiled GEMM takes from the matvec: rows at and past
+# the first such tile count (one tile per CU above 16 vectors, two up to 16),
+# a ragged last tile, and K-quants by their size; with the counts on either
+# side of 16 vectors
+@pytest.mark.parametrize("dtype,rows,cols,n,norm", [
+    (2, 32768, 96, 17, True), (8, 32770, 64, 32, False), (6, 32900, 64, 24, True), (8, 65540, 32, 9, True),
+    (2, 65540, 64, 16, False), (12, 16384, 2048, 17, True), (14, 4224, 4096, 32, False)])
+def test_batches_through_the_gemm_match_oracle(gpu, dtype, rows, cols, n, norm):
+    ctx = gpu.Ctx(512 << 20)
+    check_gemm(ctx, dtype, rows, cols, 1, n, norm)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [17, 20])
+def test_batch_logits_and_argmax_of_a_wide_head(gpu, model_dir, n):
+    """A head of 33000 rows (258 tiles, the last ragged) for more than 16
+    sessions: the GEMM's logits against each session's own step, and its
+    argmax (combined over work-groups) exactly the largest of its logits."""
+    spec = synth.ModelSpec(1, 256, 4, 2, 512, 33000, ctx_len=64, wtype=synth.Q8_0, embd_type=synth.Q8_0, wstd=0.08,
+                           seed=3)
+    m = native.Model(synth.model_file(spec, model_dir), max_ctx=32, max_sessions=n)
+    ss = [m.acquire() for _ in range(n)]
+    toks = synth.tokens(n, 9, spec.vocab)
+    ids, lg = native.decode_batch_logits(m, ss, toks, [0] * n, spec.vocab)
+    for i in range(n):
+        _, want = ss[i].forward(int(toks[i]), 0, spec.vocab)
+        assert np.all(np.abs(lg[i] - want) <= ATOL + RTOL * np.abs(want))
+        assert ids[i] == int(np.argmax(lg[i]))
+    m.close()
