@@ -341,15 +341,29 @@ int cmolhip_gemm_prepared(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, const vo
 
 } // extern "C"
 
-// Partial-sum floats a product of n vectors takes when given room, and what
-// it insists on.
-static size_t product_part_floats(const cmolhip_qtensor_t &w, int n)
-{
-    return n <= 32 ? gemv_part_floats(to_qt(w), n) : gemm_part_floats(to_qt(w), n);
-}
+// Partial-sum floats a product of n vectors insists on.
 static size_t product_part_least(const cmolhip_qtensor_t &w, int n)
 {
     return n <= 32 ? gemv_part_least(to_qt(w), n) : gemm_part_least(to_qt(w), n);
+}
+
+// Bytes of the operand and, with an RMSNorm, its sums of squares in the fixed
+// scratch of cmolhip_gemm_noalloc.
+static size_t noalloc_op_bytes(const cmolhip_qtensor_t &w, int n, bool norm, size_t *op_b = nullptr)
+{
+    const size_t o = align_up(act_bytes(w.cols, n), ALIGN);
+    if (op_b) *op_b = o;
+    return o + (norm ? align_up((size_t)n * (w.cols / 32) * 4, ALIGN) : 0);
+}
+
+// Floats it takes when given room: where cmolhip_gemm_noalloc takes the call,
+// no more than its scratch holds, so that both split k alike.
+static size_t product_part_floats(const cmolhip_qtensor_t &w, int n, bool norm)
+{
+    const size_t least = product_part_least(w, n), used = noalloc_op_bytes(w, n, norm);
+    const size_t want = std::max(least, n <= 32 ? gemv_part_floats(to_qt(w), n) : gemm_part_floats(to_qt(w), n));
+    if (used + least * 4 > NOALLOC_SCRATCH_BYTES) return want;
+    return std::min(want, (NOALLOC_SCRATCH_BYTES - used) / 4);
 }
 
 // dy[n][rows] = W . op for a prepared operand: up to 32 vectors stream the
@@ -388,7 +402,7 @@ int cmolhip_gemm_prepared_timed(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, co
     // work on this stream runs after the kernels
     const size_t mark = arena_mark(c);
     const size_t least = product_part_least(*w, n);
-    size_t pf = std::max(least, product_part_floats(*w, n));
+    size_t pf = product_part_floats(*w, n, ss != nullptr);
     float *part = nullptr;
     int rc = pf ? arena_get(c, pf, &part) : E_OK;
     if (rc == E_OOM && least < pf) {   // a small arena: fewer k ranges
@@ -427,13 +441,12 @@ int cmolhip_gemm_noalloc(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, const flo
     uint8_t *base = scratch_addr[c->device];   // resolved when c was created
     if (!base) return E_UNSUPPORTED;
     // scratch layout: operand | sum-of-squares partials | k-split partial sums
-    const size_t op_b = align_up(act_bytes(w->cols, n), ALIGN);
-    const size_t ss_b = norm_w ? align_up((size_t)n * (w->cols / 32) * 4, ALIGN) : 0;
-    const size_t least = product_part_least(*w, n);
-    if (op_b + ss_b + least * 4 > NOALLOC_SCRATCH_BYTES) return E_ARGS;   // beyond the fixed scratch
-    const size_t pf = std::min(std::max(least, product_part_floats(*w, n)), (NOALLOC_SCRATCH_BYTES - op_b - ss_b) / 4);
+    size_t op_b;
+    const size_t used = noalloc_op_bytes(*w, n, norm_w != nullptr, &op_b);
+    if (used + product_part_least(*w, n) * 4 > NOALLOC_SCRATCH_BYTES) return E_ARGS;   // beyond the fixed scratch
+    const size_t pf = product_part_floats(*w, n, norm_w != nullptr);
     float *ss = norm_w ? (float *)(base + op_b) : nullptr;
-    float *part = pf ? (float *)(base + op_b + ss_b) : nullptr;
+    float *part = pf ? (float *)(base + used) : nullptr;
     RC(cmolhip_act_prepare(c, dx, n, w->cols, w->dtype, norm_w, base, ss));
     return launch_product(c, w, base, n, ss, eps, dy, part, pf, nullptr, nullptr);
 }
