@@ -41,8 +41,10 @@
 //      accumulator of their own, so the output takes one rounding per tile.
 //      Over fp16 the A operand comes from V through ds_read_b64_tr_b16 (see
 //      attn_piece_mfw).
-// Products are exact and sums fp32.  A token whose positions fit one split is
-// finished here; otherwise each split leaves (max, sum of exp, unnormalised
+// Products are exact and sums fp32.  A masked position's weight is 0: a cached
+// V row that is not finite makes the earlier tokens that share its tile NaN
+// too, not only the later ones that attend to it.  A token whose positions fit
+// one split is finished here; otherwise each split leaves (max, sum of exp, unnormalised
 // output) in the partial format of attn_split and k_attn_merge_wave combines
 // them.
 //
