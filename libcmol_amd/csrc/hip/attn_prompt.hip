@@ -41,12 +41,14 @@
 //      accumulator of their own, so the output takes one rounding per tile.
 //      Over fp16 the A operand comes from V through ds_read_b64_tr_b16 (see
 //      attn_piece_mfw).
-// Products are exact and sums fp32.  A masked position's weight is 0: a cached
-// V row that is not finite makes the earlier tokens that share its tile NaN
-// too, not only the later ones that attend to it.  A token whose positions fit
-// one split is finished here; otherwise each split leaves (max, sum of exp, unnormalised
-// output) in the partial format of attn_split and k_attn_merge_wave combines
-// them.
+// Products are exact and sums fp32.  A masked position's weight is 0, so a
+// cached V row that is not finite would make the earlier tokens that share its
+// tile NaN (0 * inf); a work-group whose outputs are not all finite walks its
+// split again with such rows taken apart, and only the rows that attend to one
+// are NaN, as in a decode of the tokens one by one.  A token whose positions
+// fit one split is finished here; otherwise each split leaves (max, sum of
+// exp, unnormalised output) in the partial format of attn_split and
+// k_attn_merge_wave combines them.
 //
 // Bound: latency and the causal imbalance.  Per tile a wave has 1024 (fp16)
 // or 768 (fp32) cycles of the matrix pipe and about 640 of softmax VALU in a
@@ -110,8 +112,36 @@ __global__ __launch_bounds__(256) void k_kv_hilo(AttnArgs a, int last, _Float16 
     }
 }
 
+// Takes the values that are not finite out of the V part `v` of a half's
+// staged tile, by the half's 256 threads (t) and within two barriers of the
+// work-group: they become 0 and bad[position] is set.  `on`: the half has a tile.
 template <int DH, bool F16>
-__global__ __launch_bounds__(PA_NT) __attribute__((amdgpu_waves_per_eu(2)))
+__device__ __forceinline__ void pa_take_apart(uint8_t *v, uint8_t *bad, int t, bool on)
+{
+    constexpr int TP = F16 ? 64 : KVT_POS, CHUNKS = TP * DH * 2 / 16;   // 16-byte pieces (fp32: high ones)
+    if (t < TP) bad[t] = 0;
+    __syncthreads();
+    for (int q = t; on && q < CHUNKS; q += 256) {
+        // fp32: piece (dimension tile, lane), its high half here and its low one 1 KiB on
+        f16x8 *p = (f16x8 *)(v + (F16 ? q * 16 : (q >> 6) * 2048 + (q & 63) * 16));
+        f16x8 x = *p;
+        bool any = false;
+        for (int e = 0; e < 8; e++) {
+            if ((__builtin_bit_cast(uint16_t, (_Float16)x[e]) & 0x7c00) != 0x7c00) continue;
+            const int g = (q & 63) >> 4;
+            bad[F16 ? q * 16 / (2 * DH) : 4 * g + (e & 3) + 16 * (e >> 2)] = 1;
+            x[e] = 0;
+            if (!F16) ((_Float16 *)p)[512 + e] = 0;
+            any = true;
+        }
+        if (any) *p = x;
+    }
+    __syncthreads();
+}
+
+// (d_head 64: LDS lets a CU hold two work-groups, so 128 VGPRs)
+template <int DH, bool F16>
+__global__ __launch_bounds__(PA_NT) __attribute__((amdgpu_waves_per_eu(DH == 64 ? 4 : 2)))
 void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
 {
 #pragma clang fp contract(off)
@@ -124,6 +154,7 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
     constexpr int PIECES = TILE / 1024 / 4;           // fp32: pieces per wave
     constexpr int DH2 = DT / 2;                       // dimension tiles each half finishes
     extern __shared__ __attribute__((aligned(256))) uint8_t smem_p[];   // [stage][half][TILE]
+    __shared__ uint8_t badrow[2][TP];   // V rows of the halves' tiles that are not finite (see apart)
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, col = lane & 15;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), half = wid >> 2, w4 = wid & 3;
@@ -197,142 +228,166 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
     const int lim = min(L, pb);   // visible positions of this split: pa .. lim-1
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 o[DT], o2[DT];   // o2: products with a low part, times 2048
-#pragma unroll
-    for (int t = 0; t < DT; t++) {
-        o[t] = zero4;
-        o2[t] = zero4;
-    }
-    // mk = -m c2; a row with no visible position yet (m = -inf) has weights 0
-    float m = -INFINITY, mk = 0.0f, lsum = 0.0f;
+    float m, mk, lsum;     // mk = -m c2; a row with no visible position yet (m = -inf) has weights 0
+    f32x4 r[DH2];          // the dimensions of this lane's row that its half finishes
+    float mm, ls;
     // fp16: transposing reads, this lane's bytes of row 4g + col/4 (+ 16 per c)
     // of dimension tile t at vaddr ^ 32t
     const int vr = 4 * g + (col >> 2);
     const uint32_t vaddr = (uint32_t)(vr * (2 * DH) + 32 * (DH == 128 ? vr & 7 : (vr >> 1) & 3) + 8 * (col & 3));
 
-    int st = 0;
-    for (int pp = pa; pp < pb; pp += 2 * TP, st ^= 1) {
-        const int p0 = pp + half * TP;   // this half's tile
-        // the tiles have landed and every wave is done with the other stage
-        __builtin_amdgcn_s_waitcnt(WAITCNT_VM_LGKM0(0));
-        __syncthreads();
-        if (p0 + 2 * TP < pb) issue(st ^ 1, p0 + 2 * TP);
-        if (p0 >= pb) continue;          // (the last pair may be one tile)
-        const uint8_t *ks_ = smem_p + (st * 2 + half) * TILE, *vs_ = ks_ + KB;
-        // ---- scores: sc[c][i] = position p0 + 16c + 4g + i of this lane's row
-        float sc[CT][4];
+    // Masked positions are in the products with weight 0, so a V row that is not
+    // finite leaves NaN (0 * inf) in the rows that do not see it, too.  Where an
+    // output is not finite the walk is done again with such rows taken apart.
+    for (bool apart = false;; apart = true) {
+        m = -INFINITY;
+        mk = 0.0f;
+        lsum = 0.0f;
 #pragma unroll
-        for (int c = 0; c < CT; c++) {
-            f32x4 s1 = zero4, s2 = zero4;
-#pragma unroll
-            for (int s = 0; s < KS; s++) {
-                if constexpr (F16) {
-                    const f16x8 kf = *(const f16x8 *)(ks_ + (c * KS + s) * 1024 + lane * 16);
-                    s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[s], s1, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[s], s2, 0, 0, 0);
-                } else {
-                    const f16x8 kh = *(const f16x8 *)(ks_ + (c * KS + s) * 2048 + lane * 16);
-                    const f16x8 kl = *(const f16x8 *)(ks_ + (c * KS + s) * 2048 + 1024 + lane * 16);
-                    s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[s], s1, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[s], s2, 0, 0, 0);
-                    s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[s], s2, 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) sc[c][i] = fmaf(s2[i], 1.0f / 2048.0f, s1[i]);
+        for (int t = 0; t < DT; t++) {
+            o[t] = zero4;
+            o2[t] = zero4;
         }
-        if (p0 + TP > whole) {   // uniform: the causal edge and the split's end
+        int st = 0;
+        for (int pp = pa; pp < pb; pp += 2 * TP, st ^= 1) {
+            const int p0 = pp + half * TP;   // this half's tile
+            // the tiles have landed and every wave is done with the other stage
+            __builtin_amdgcn_s_waitcnt(WAITCNT_VM_LGKM0(0));
+            __syncthreads();
+            if (p0 + 2 * TP < pb) issue(st ^ 1, p0 + 2 * TP);
+            if (apart) pa_take_apart<DH, F16>(smem_p + (st * 2 + half) * TILE + KB, badrow[half], tid & 255, p0 < pb);
+            if (p0 >= pb) continue;          // (the last pair may be one tile)
+            const uint8_t *ks_ = smem_p + (st * 2 + half) * TILE, *vs_ = ks_ + KB;
+            // ---- scores: sc[c][i] = position p0 + 16c + 4g + i of this lane's row
+            float sc[CT][4];
+#pragma unroll
+            for (int c = 0; c < CT; c++) {
+                f32x4 s1 = zero4, s2 = zero4;
+#pragma unroll
+                for (int s = 0; s < KS; s++) {
+                    if constexpr (F16) {
+                        const f16x8 kf = *(const f16x8 *)(ks_ + (c * KS + s) * 1024 + lane * 16);
+                        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[s], s1, 0, 0, 0);
+                        s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[s], s2, 0, 0, 0);
+                    } else {
+                        const f16x8 kh = *(const f16x8 *)(ks_ + (c * KS + s) * 2048 + lane * 16);
+                        const f16x8 kl = *(const f16x8 *)(ks_ + (c * KS + s) * 2048 + 1024 + lane * 16);
+                        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[s], s1, 0, 0, 0);
+                        s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[s], s2, 0, 0, 0);
+                        s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[s], s2, 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) sc[c][i] = fmaf(s2[i], 1.0f / 2048.0f, s1[i]);
+            }
+            if (p0 + TP > whole) {   // uniform: the causal edge and the split's end
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (p0 + 16 * c + 4 * g + i >= lim) sc[c][i] = -INFINITY;
+            }
+            if (apart) {
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (badrow[half][16 * c + 4 * g + i] && p0 + 16 * c + 4 * g + i < lim) sc[c][i] = __builtin_nanf("");
+            }
+            // ---- online softmax of the row (its scores: lanes col + 16 g) ----
+            float mx = sc[0][0];
 #pragma unroll
             for (int c = 0; c < CT; c++)
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (p0 + 16 * c + 4 * g + i >= lim) sc[c][i] = -INFINITY;
-        }
-        // ---- online softmax of the row (its scores: lanes col + 16 g) ----
-        float mx = sc[0][0];
+                for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[c][i]);
+            if (__ballot(mx > m + lazy)) {
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                const float mn = fmaxf(m, mx);
+                const float mref = mn == -INFINITY ? 0.0f : mn;
+                const float al = mn == m ? 1.0f : __builtin_amdgcn_exp2f((m - mref) * c2);
+                m = mn;
+                mk = -mref * c2;
+                lsum *= al;
 #pragma unroll
-        for (int c = 0; c < CT; c++)
+                for (int t = 0; t < DT; t++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[c][i]);
-        if (__ballot(mx > m + lazy)) {
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float mn = fmaxf(m, mx);
-            const float mref = mn == -INFINITY ? 0.0f : mn;
-            const float al = mn == m ? 1.0f : __builtin_amdgcn_exp2f((m - mref) * c2);
-            m = mn;
-            mk = -mref * c2;
-            lsum *= al;
+                    for (int i = 0; i < 4; i++) {
+                        o[t][i] *= al;
+                        o2[t][i] *= al;
+                    }
+                }
+            }
+            f16x8 ph[CT / 2], pl[CT / 2];
 #pragma unroll
-            for (int t = 0; t < DT; t++) {
+            for (int c = 0; c < CT; c++) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    o[t][i] *= al;
-                    o2[t][i] *= al;
+                    const float e = __builtin_amdgcn_exp2f(fmaf(sc[c][i], c2, mk));
+                    lsum += e;
+                    const _Float16 hi = (_Float16)e;
+                    ph[c >> 1][4 * (c & 1) + i] = hi;
+                    pl[c >> 1][4 * (c & 1) + i] = (_Float16)((e - (float)hi) * 2048.0f);
+                }
+            }
+            // ---- O^T += V^T P^T: k-step k covers positions 32k + 4g .. +3 and 32k + 16 + 4g .. +3
+#pragma unroll
+            for (int k = 0; k < CT / 2; k++) {
+#pragma unroll
+                for (int t = 0; t < DT; t++) {
+                    if constexpr (F16) {
+                        typedef short s16x4 __attribute__((ext_vector_type(4)));
+                        typedef __attribute__((address_space(3))) s16x4 ls16x4;
+                        const uint8_t *src = vs_ + 32 * k * (2 * DH) + (vaddr ^ (32u * t));
+                        const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4 *)src);
+                        const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4 *)(src + 16 * (2 * DH)));
+                        const f16x8 vf = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
+                        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[k], o[t], 0, 0, 0);
+                        o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[k], o2[t], 0, 0, 0);
+                    } else {
+                        const f16x8 vh = *(const f16x8 *)(vs_ + t * 2048 + lane * 16);
+                        const f16x8 vl = *(const f16x8 *)(vs_ + t * 2048 + 1024 + lane * 16);
+                        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[k], o[t], 0, 0, 0);
+                        o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[k], o2[t], 0, 0, 0);
+                        o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[k], o2[t], 0, 0, 0);
+                    }
                 }
             }
         }
-        f16x8 ph[CT / 2], pl[CT / 2];
-#pragma unroll
-        for (int c = 0; c < CT; c++) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float e = __builtin_amdgcn_exp2f(fmaf(sc[c][i], c2, mk));
-                lsum += e;
-                const _Float16 hi = (_Float16)e;
-                ph[c >> 1][4 * (c & 1) + i] = hi;
-                pl[c >> 1][4 * (c & 1) + i] = (_Float16)((e - (float)hi) * 2048.0f);
-            }
-        }
-        // ---- O^T += V^T P^T: k-step k covers positions 32k + 4g .. +3 and 32k + 16 + 4g .. +3
-#pragma unroll
-        for (int k = 0; k < CT / 2; k++) {
-#pragma unroll
-            for (int t = 0; t < DT; t++) {
-                if constexpr (F16) {
-                    typedef short s16x4 __attribute__((ext_vector_type(4)));
-                    typedef __attribute__((address_space(3))) s16x4 ls16x4;
-                    const uint8_t *src = vs_ + 32 * k * (2 * DH) + (vaddr ^ (32u * t));
-                    const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4 *)src);
-                    const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4 *)(src + 16 * (2 * DH)));
-                    const f16x8 vf = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo4, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
-                    o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[k], o[t], 0, 0, 0);
-                    o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[k], o2[t], 0, 0, 0);
-                } else {
-                    const f16x8 vh = *(const f16x8 *)(vs_ + t * 2048 + lane * 16);
-                    const f16x8 vl = *(const f16x8 *)(vs_ + t * 2048 + 1024 + lane * 16);
-                    o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[k], o[t], 0, 0, 0);
-                    o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[k], o2[t], 0, 0, 0);
-                    o2[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[k], o2[t], 0, 0, 0);
-                }
-            }
-        }
-    }
 
-    // ---- the halves meet: half 0 finishes the first DT / 2 dimension tiles of
-    // each row, half 1 the others
+        // ---- the halves meet: half 0 finishes the first DT / 2 dimension tiles of
+        // each row, half 1 the others
 #pragma unroll
-    for (int t = 0; t < DT; t++) o[t] += o2[t] * (1.0f / 2048.0f);
-    lsum += __shfl_xor(lsum, 16, 64);
-    lsum += __shfl_xor(lsum, 32, 64);
-    f32x4 *xo = (f32x4 *)smem_p;                        // [half][wave][DT / 2][lane]
-    float *xm = (float *)(smem_p + 8 * DH2 * 64 * 16);   // [half][row] m, then [half][row] l
-    __syncthreads();
+        for (int t = 0; t < DT; t++) o[t] += o2[t] * (1.0f / 2048.0f);
+        lsum += __shfl_xor(lsum, 16, 64);
+        lsum += __shfl_xor(lsum, 32, 64);
+        f32x4 *xo = (f32x4 *)smem_p;                        // [half][wave][DT / 2][lane]
+        float *xm = (float *)(smem_p + 8 * DH2 * 64 * 16);   // [half][row] m, then [half][row] l
+        __syncthreads();
 #pragma unroll
-    for (int t = 0; t < DH2; t++) xo[((half * 4 + w4) * DH2 + t) * 64 + lane] = half ? o[t] : o[DH2 + t];
-    if (g == 0) {
-        xm[half * 64 + ar] = m;
-        xm[128 + half * 64 + ar] = lsum;
-    }
-    __syncthreads();
-    const float m1 = xm[(half ^ 1) * 64 + ar], l1 = xm[128 + (half ^ 1) * 64 + ar];
-    const float mm = fmaxf(m, m1), mref = mm == -INFINITY ? 0.0f : mm;
-    const float f0 = __builtin_amdgcn_exp2f((m - mref) * c2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * c2);
-    const float ls = lsum * f0 + l1 * f1;
-    f32x4 r[DH2];
+        for (int t = 0; t < DH2; t++) xo[((half * 4 + w4) * DH2 + t) * 64 + lane] = half ? o[t] : o[DH2 + t];
+        if (g == 0) {
+            xm[half * 64 + ar] = m;
+            xm[128 + half * 64 + ar] = lsum;
+        }
+        __syncthreads();
+        const float m1 = xm[(half ^ 1) * 64 + ar], l1 = xm[128 + (half ^ 1) * 64 + ar];
+        mm = fmaxf(m, m1);
+        const float mref = mm == -INFINITY ? 0.0f : mm;
+        const float f0 = __builtin_amdgcn_exp2f((m - mref) * c2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * c2);
+        ls = lsum * f0 + l1 * f1;
 #pragma unroll
-    for (int t = 0; t < DH2; t++) {
-        const f32x4 mine = half ? o[DH2 + t] : o[t], other = xo[(((half ^ 1) * 4 + w4) * DH2 + t) * 64 + lane];
-        r[t] = mine * f0 + other * f1;
+        for (int t = 0; t < DH2; t++) {
+            const f32x4 mine = half ? o[DH2 + t] : o[t], other = xo[(((half ^ 1) * 4 + w4) * DH2 + t) * 64 + lane];
+            r[t] = mine * f0 + other * f1;
+        }
+        bool fin = true;
+#pragma unroll
+        for (int t = 0; t < DH2; t++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) fin = fin && fabsf(r[t][i]) < INFINITY;
+        if (apart || !__syncthreads_or(!fin)) break;
+        if (pa + half * TP < pb) issue(0, pa + half * TP);
     }
 
     // ---- outputs: lane (col, g) holds dimensions 16 (DH2 half + t) + 4g + i of its row
