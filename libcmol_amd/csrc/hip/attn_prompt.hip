@@ -63,6 +63,7 @@
 // rows, each K/V fragment read once for two row groups (four waves): 70
 // against 68 us at 2048 tokens over fp16, 28.8 against 26.8 at 512.
 #include "attn_impl.h"
+#include "lds_limit.h"
 
 constexpr float PA_LAZY = 2.0f;      // log2: weights stay below 4
 constexpr int PA_NT = 512;
@@ -448,10 +449,12 @@ template <int DH, bool F16>
 static int launch_dh(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s)
 {
     constexpr int LDS = 4 * 64 * DH * 4;   // two stages of two tiles (64 positions fp16 or 32 high/low, K and V)
-    static const bool lds_ok =
-        hipFuncSetAttribute((const void *)k_attn_prompt<DH, F16>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) ==
-        hipSuccess;
-    if (!lds_ok) return -4;
+    static LdsLimit limit;
+    const bool ok = limit.raise(current_device(), [] {
+        return hipFuncSetAttribute((const void *)k_attn_prompt<DH, F16>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) ==
+               hipSuccess;
+    });
+    if (!ok) return -4;
     const int QT = 64 / (a.n_heads / a.n_kv);
     const int tiles = (a.max_ctx + KVT_POS - 1) / KVT_POS;
     if constexpr (!F16)

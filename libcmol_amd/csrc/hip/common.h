@@ -23,6 +23,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 enum { DT_F32 = 0, DT_F16 = 1, DT_Q4_0 = 2, DT_Q5_0 = 6, DT_Q8_0 = 8, DT_Q4_K = 12, DT_Q6_K = 14 };
 
+// The calling thread's device, -1 if unknown.
+static inline int current_device()
+{
+    int d = -1;
+    if (hipGetDevice(&d) == hipSuccess) return d;
+    (void)hipGetLastError();
+    return -1;
+}
+
 // Global-memory view of a generic pointer: accesses through the result
 // compile to global_* instructions.  Used where the compiler cannot infer the
 // address space itself (pointers read from memory), which would otherwise

@@ -4,10 +4,10 @@
 #pragma once
 #include "common.h"
 #include "kernels.h"
+#include "lds_limit.h"
 
 #include <hip/hip_ext.h>
 
-#include <atomic>
 #include <cstdlib>
 
 // k-split finish of the batched matvec (gemv.hip): sums the `splits`
@@ -1183,16 +1183,12 @@ static int launch_gemv_b16_nw(const GemvArgs &a, const Gb16Shape &p, hipStream_t
 {
     constexpr int U = (DT == DT_Q8_0) ? 6 : 8;
     const size_t lds = (size_t)p.sq * 4 * 2048 + 64;
-    // set once; a refusal (e.g. inside a stream capture) is retried on the
-    // next launch rather than remembered (decode threads of several sessions
-    // may get here at once: the flag is atomic, the attribute call idempotent)
-    static std::atomic<bool> lds_ok{false};
-    if (!lds_ok.load(std::memory_order_relaxed)) {
-        if (hipFuncSetAttribute((const void *)k_gemv_b16<DT, U, EPI, NWB>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
-            return -6;
-        lds_ok.store(true, std::memory_order_relaxed);
-    }
+    static LdsLimit limit;
+    const bool ok = limit.raise(current_device(), [] {
+        return hipFuncSetAttribute((const void *)k_gemv_b16<DT, U, EPI, NWB>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   160 * 1024) == hipSuccess;
+    });
+    if (!ok) return -6;
     const long blocks = (long)((p.rblocks * p.splits + 7) / 8) * 8 * p.groups;
     const bool split = p.splits > 1;
     if (a.ev_start)
