@@ -115,7 +115,8 @@ __global__ __launch_bounds__(256) void k_kv_hilo(AttnArgs a, int last, _Float16 
 
 // Takes the values that are not finite out of the V part `v` of a half's
 // staged tile, by the half's 256 threads (t) and within two barriers of the
-// work-group: they become 0 and bad[position] is set.  `on`: the half has a tile.
+// work-group: they become 0 and bad[position] is set.  `on`: the half has a tile
+// with masked positions.
 template <int DH, bool F16>
 __device__ __forceinline__ void pa_take_apart(uint8_t *v, uint8_t *bad, int t, bool on)
 {
@@ -230,8 +231,6 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
     const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 o[DT], o2[DT];   // o2: products with a low part, times 2048
     float m, mk, lsum;     // mk = -m c2; a row with no visible position yet (m = -inf) has weights 0
-    f32x4 r[DH2];          // the dimensions of this lane's row that its half finishes
-    float mm, ls;
     // fp16: transposing reads, this lane's bytes of row 4g + col/4 (+ 16 per c)
     // of dimension tile t at vaddr ^ 32t
     const int vr = 4 * g + (col >> 2);
@@ -239,7 +238,8 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
 
     // Masked positions are in the products with weight 0, so a V row that is not
     // finite leaves NaN (0 * inf) in the rows that do not see it, too.  Where an
-    // output is not finite the walk is done again with such rows taken apart.
+    // output is not finite the walk is done again with such rows taken apart, and
+    // the outputs written again (the vote on it is off the way to the first ones).
     for (bool apart = false;; apart = true) {
         m = -INFINITY;
         mk = 0.0f;
@@ -256,7 +256,9 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
             __builtin_amdgcn_s_waitcnt(WAITCNT_VM_LGKM0(0));
             __syncthreads();
             if (p0 + 2 * TP < pb) issue(st ^ 1, p0 + 2 * TP);
-            if (apart) pa_take_apart<DH, F16>(smem_p + (st * 2 + half) * TILE + KB, badrow[half], tid & 255, p0 < pb);
+            if (__builtin_expect(apart && pp + 2 * TP > whole, 0))   // (alike in both halves: it has barriers)
+                pa_take_apart<DH, F16>(smem_p + (st * 2 + half) * TILE + KB, badrow[half], tid & 255,
+                                       p0 < pb && p0 + TP > whole);
             if (p0 >= pb) continue;          // (the last pair may be one tile)
             const uint8_t *ks_ = smem_p + (st * 2 + half) * TILE, *vs_ = ks_ + KB;
             // ---- scores: sc[c][i] = position p0 + 16c + 4g + i of this lane's row
@@ -287,13 +289,13 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
                         if (p0 + 16 * c + 4 * g + i >= lim) sc[c][i] = -INFINITY;
-            }
-            if (apart) {
+                if (__builtin_expect(apart, 0)) {
 #pragma unroll
-                for (int c = 0; c < CT; c++)
+                    for (int c = 0; c < CT; c++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (badrow[half][16 * c + 4 * g + i] && p0 + 16 * c + 4 * g + i < lim) sc[c][i] = __builtin_nanf("");
+                        for (int i = 0; i < 4; i++)
+                            if (badrow[half][16 * c + 4 * g + i] && p0 + 16 * c + 4 * g + i < lim) sc[c][i] = __builtin_nanf("");
+                }
             }
             // ---- online softmax of the row (its scores: lanes col + 16 g) ----
             float mx = sc[0][0];
@@ -356,72 +358,81 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
             }
         }
 
+        // The addresses below start from copies that the compiler takes as new
+        // in each walk: it would compute them all before the first one and hold
+        // them in registers, or spill them, during it.
+        int ln = lane, tok = at, hd = ah, len = L;
+        asm volatile("" : "+v"(ln), "+v"(tok), "+v"(hd), "+v"(len));
+        const int gg = ln >> 4, row = 16 * w4 + (ln & 15);
         // ---- the halves meet: half 0 finishes the first DT / 2 dimension tiles of
         // each row, half 1 the others
 #pragma unroll
         for (int t = 0; t < DT; t++) o[t] += o2[t] * (1.0f / 2048.0f);
+        f32x4 z = zero4;   // NaN where an output of the lane is not finite
+#pragma unroll
+        for (int t = 0; t < DT; t++) z += o[t] * 0.0f;
         lsum += __shfl_xor(lsum, 16, 64);
         lsum += __shfl_xor(lsum, 32, 64);
         f32x4 *xo = (f32x4 *)smem_p;                        // [half][wave][DT / 2][lane]
-        float *xm = (float *)(smem_p + 8 * DH2 * 64 * 16);   // [half][row] m, then [half][row] l
+        float *xm = (float *)(smem_p + 8 * DH2 * 64 * 16);   // [half][row] m, then [half][row] l, then a vote per wave
+        const bool fin = __ballot(!(z[0] + z[1] + z[2] + z[3] == 0.0f)) == 0;
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < DH2; t++) xo[((half * 4 + w4) * DH2 + t) * 64 + lane] = half ? o[t] : o[DH2 + t];
-        if (g == 0) {
-            xm[half * 64 + ar] = m;
-            xm[128 + half * 64 + ar] = lsum;
+        for (int t = 0; t < DH2; t++) xo[((half * 4 + w4) * DH2 + t) * 64 + ln] = half ? o[t] : o[DH2 + t];
+        if (gg == 0) {
+            xm[half * 64 + row] = m;
+            xm[128 + half * 64 + row] = lsum;
         }
+        if (ln == 0) xm[256 + wid] = fin ? 0.0f : 1.0f;
         __syncthreads();
-        const float m1 = xm[(half ^ 1) * 64 + ar], l1 = xm[128 + (half ^ 1) * 64 + ar];
-        mm = fmaxf(m, m1);
-        const float mref = mm == -INFINITY ? 0.0f : mm;
+        const float m1 = xm[(half ^ 1) * 64 + row], l1 = xm[128 + (half ^ 1) * 64 + row];
+        const float mm = fmaxf(m, m1), mref = mm == -INFINITY ? 0.0f : mm;
         const float f0 = __builtin_amdgcn_exp2f((m - mref) * c2), f1 = __builtin_amdgcn_exp2f((m1 - mref) * c2);
-        ls = lsum * f0 + l1 * f1;
+        const float ls = lsum * f0 + l1 * f1;
+        f32x4 r[DH2];
 #pragma unroll
         for (int t = 0; t < DH2; t++) {
-            const f32x4 mine = half ? o[DH2 + t] : o[t], other = xo[(((half ^ 1) * 4 + w4) * DH2 + t) * 64 + lane];
-            r[t] = mine * f0 + other * f1;
+            const f32x4 own = half ? o[DH2 + t] : o[t], other = xo[(((half ^ 1) * 4 + w4) * DH2 + t) * 64 + ln];
+            r[t] = own * f0 + other * f1;
         }
-        bool fin = true;
-#pragma unroll
-        for (int t = 0; t < DH2; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) fin = fin && fabsf(r[t][i]) < INFINITY;
-        if (apart || !__syncthreads_or(!fin)) break;
-        if (pa + half * TP < pb) issue(0, pa + half * TP);
-    }
 
-    // ---- outputs: lane (col, g) holds dimensions 16 (DH2 half + t) + 4g + i of its row
-    const int nact = (L + a.split - 1) / a.split;
-    if (!arow || sp >= nact) return;   // no positions of this token here
-    const int v = vb + at, d0 = 16 * DH2 * half + 4 * g;
-    if (nact == 1) {
-        const float inv = 1.0f / ls;
-        const int k0 = (kvh * G + ah) * DH + d0;
+        // ---- outputs: lane (col, g) holds dimensions 16 (DH2 half + t) + 4g + i of its row
+        const int nact = (len + a.split - 1) / a.split;
+        const bool mine = arow && sp < nact;   // (else no positions of this token here)
+        const int v = vb + tok, d0 = 16 * DH2 * half + 4 * gg;
+        if (mine && nact == 1) {
+            const float inv = 1.0f / ls;
+            const int k0 = (kvh * G + hd) * DH + d0;
 #pragma unroll
-        for (int t = 0; t < DH2; t += 2) {
-            const f32x4 x0 = r[t] * inv, x1 = r[t + 1] * inv;
-            const int k = k0 + 16 * t;
-            if (a.out) {
-                *(f32x4 *)(a.out + (size_t)v * a.out_stride + k) = x0;
-                *(f32x4 *)(a.out + (size_t)v * a.out_stride + k + 16) = x1;
+            for (int t = 0; t < DH2; t += 2) {
+                const f32x4 x0 = r[t] * inv, x1 = r[t + 1] * inv;
+                const int k = k0 + 16 * t;
+                if (a.out) {
+                    *(f32x4 *)(a.out + (size_t)v * a.out_stride + k) = x0;
+                    *(f32x4 *)(a.out + (size_t)v * a.out_stride + k + 16) = x1;
+                }
+                if (!a.next.q) continue;
+                if (a.next.dt == DT_Q8_0) {
+                    act_put4(a.next, v, k, x0);
+                    act_put4(a.next, v, k + 16, x1);
+                } else {
+                    act_put8(a.next, v, k >> 5, gg, k, k + 16, x0, x1);
+                }
             }
-            if (!a.next.q) continue;
-            if (a.next.dt == DT_Q8_0) {
-                act_put4(a.next, v, k, x0);
-                act_put4(a.next, v, k + 16, x1);
-            } else {
-                act_put8(a.next, v, k >> 5, g, k, k + 16, x0, x1);
+        } else if (mine) {
+            const size_t sb = (((size_t)v * a.n_kv + kvh) * a.max_splits + sp) * G + hd;
+#pragma unroll
+            for (int t = 0; t < DH2; t++) *(f32x4 *)&a.po[sb * DH + d0 + 16 * t] = r[t];
+            if (gg == 0 && half == 0) {
+                a.pm[sb] = mm * scale;   // natural units, as the merge reads them
+                a.pl[sb] = ls;
             }
         }
-    } else {
-        const size_t sb = (((size_t)v * a.n_kv + kvh) * a.max_splits + sp) * G + ah;
-#pragma unroll
-        for (int t = 0; t < DH2; t++) *(f32x4 *)&a.po[sb * DH + d0 + 16 * t] = r[t];
-        if (g == 0 && half == 0) {
-            a.pm[sb] = mm * scale;   // natural units, as the merge reads them
-            a.pl[sb] = ls;
-        }
+
+        const f32x4 v0 = *(const f32x4 *)&xm[256], v1 = *(const f32x4 *)&xm[260], vs = v0 + v1;
+        if (__builtin_expect(apart || vs[0] + vs[1] + vs[2] + vs[3] == 0.0f, 1)) break;
+        __syncthreads();
+        if (pa + half * TP < pb) issue(0, pa + half * TP);
     }
 }
 
