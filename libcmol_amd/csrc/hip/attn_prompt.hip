@@ -65,6 +65,8 @@
 #include "attn_impl.h"
 #include "lds_limit.h"
 
+#include <algorithm>
+
 constexpr float PA_LAZY = 2.0f;      // log2: weights stay below 4
 constexpr int PA_NT = 512;
 constexpr int KVT_POS = 32;          // positions per tile of the high/low copy
@@ -476,24 +478,45 @@ static int launch_dh(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s
     return a.max_splits > 1 ? launch_attn_merge_wave(a, s) : 0;
 }
 
-int launch_attn_prompt(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s)
+// Work-groups of one round: LDS lets a CU hold two at d_head 64, one at 128.
+static long prompt_round(int d_head) { return (long)prompt_cus() * (128 / d_head); }
+
+// Work-groups of n tokens per split.
+static long prompt_blocks(int n, int n_heads, int n_kv)
+{
+    const int QT = 64 / (n_heads / n_kv);
+    return (long)n_kv * ((n + QT - 1) / QT);
+}
+
+size_t attn_prompt_rows(int cap, int n_heads, int n_kv, int d_head, int max_ctx, int split)
+{
+    size_t m = 0;
+    for (int n = 1; n <= cap; n++) {
+        const long s = std::min((long)attn_max_splits(max_ctx, split), prompt_round(d_head) / prompt_blocks(n, n_heads, n_kv));
+        if (s > 1) m = std::max(m, (size_t)n * n_heads * s);
+    }
+    return m;
+}
+
+int launch_attn_prompt(const AttnArgs &a, size_t part_rows, _Float16 *kv_hl, int last, hipStream_t s)
 {
     const int G = a.n_heads / a.n_kv;
     if (G < 1 || G > 8 || a.n_heads % a.n_kv || a.n < 1 || (a.d_head != 64 && a.d_head != 128)) return -4;
     if (a.split < 64 || a.split % 64 || a.max_splits > ATT_MAX_MERGE) return -4;
     if ((!a.kv_f16 && !kv_hl) || last < 1 || last > a.max_ctx) return -4;
     // the pass's split: the planned one doubled until the grid fits one round
-    // of the work-groups that LDS lets a CU hold (two at d_head 64, one at
-    // 128); blocks that alone exceed it run unsplit, longest first.  At 16/4
+    // of the work-groups and the partials their buffers (one split has none);
+    // blocks that alone exceed a round run unsplit, longest first.  At 16/4
     // heads of 128 over fp16, with merge: 512 tokens behind 1300 positions 35
     // us in 2 splits (taken), 44 in 4, 43 in 1; 188 behind 1812 24 in 4
-    // (taken), 30 in 8.  Fewer splits than planned always fit the partial
-    // buffers.
+    // (taken), 30 in 8.
     AttnArgs b = a;
-    const long blocks = (long)a.n_kv * ((a.n + 64 / G - 1) / (64 / G));
-    while (b.split < last && blocks * ((last + b.split - 1) / b.split) > (long)prompt_cus() * (128 / a.d_head))
+    const long blocks = prompt_blocks(a.n, a.n_heads, a.n_kv);
+    auto splits = [&] { return (last + b.split - 1) / b.split; };
+    while (b.split < last &&
+           (blocks * splits() > prompt_round(a.d_head) || (size_t)a.n * a.n_heads * splits() > part_rows))
         b.split *= 2;
-    b.max_splits = (last + b.split - 1) / b.split;
+    b.max_splits = splits();
     int rc;
     if (a.kv_f16) rc = a.d_head == 128 ? launch_dh<128, true>(b, kv_hl, last, s) : launch_dh<64, true>(b, kv_hl, last, s);
     else rc = a.d_head == 128 ? launch_dh<128, false>(b, kv_hl, last, s) : launch_dh<64, false>(b, kv_hl, last, s);

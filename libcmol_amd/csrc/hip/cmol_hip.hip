@@ -616,11 +616,13 @@ struct Prefill {
     _Float16 *op_qkv = nullptr, *op_o = nullptr, *op_gu = nullptr, *op_dn = nullptr,
              *op_lm = nullptr;
     float *ss_a = nullptr, *ss_b = nullptr;   // [cap][d]
-    float *pm = nullptr, *pl = nullptr, *po = nullptr;
     float *qkv_raw = nullptr;                 // QK-norm models: [cap][d + 2 kvd]
     _Float16 *kv_hl = nullptr;                // prompt attention: high/low f16 copy of one layer's cache
-    float *part = nullptr;                    // split-K partial sums of the prompt GEMMs
+    // split-K partial sums of the GEMMs and split partials of the attention,
+    // one stage after another in the same room
+    float *part = nullptr;
     size_t part_cap = 0;                      // floats at part
+    size_t part_rows = 0;                     // attention partials it holds (d_head + 2 floats each)
     int32_t *h_steps = nullptr;               // pinned [cap][3]
     int32_t *h_slots = nullptr;               // pinned [cap]
     std::mutex mu;
@@ -666,12 +668,11 @@ bool prompt_attn_fits(const cmolhip_hparams_t &h)
 }
 
 // Positions per attention work-group in a prompt pass: the split kernels
-// take at most 16 splits of at least 1024 positions; the prompt kernel, whose
+// take at most 16 splits of at least 1024 positions; the prompt kernel (pk), whose
 // work-groups already share K/V across 64 query rows, at most 32 splits of
 // at least 256 (more work-groups for a pass over a short prefix).
-int prefill_split(const cmolhip_hparams_t &h)
+int prefill_split(const cmolhip_hparams_t &h, bool pk)
 {
-    const bool pk = prompt_attn_fits(h);
     int s = (h.max_ctx + (pk ? 31 : 15)) / (pk ? 32 : 16);
     s = (s + 63) / 64 * 64;
     const int lo = pk ? 256 : 1024;
@@ -981,13 +982,29 @@ size_t prefill_part_floats(const cmolhip_model_desc_t *d)
     return m;
 }
 
+// Floats of the room in which the stages of a prompt pass leave partials: what
+// its GEMMs' k ranges and its attention's splits can use, whichever is more,
+// and at most four k ranges of q|k|v and the splits of 1024 positions (at most
+// 16; prompt attention over fp32 caches: of 256, at most 32) at the full pass
+// length, which models have always been sized for.  Shorter of room, both take
+// fewer.
+size_t prefill_part_cap(const cmolhip_model_desc_t *d)
+{
+    const cmolhip_hparams_t &h = d->hp;
+    const int cap = prefill_cap(h), row = h.d_head + 2;
+    const int ms = attn_max_splits(h.max_ctx, prefill_split(h, prompt_attn_fits(h) && !h.kv_f16));
+    const size_t full = (size_t)cap * h.n_heads * ms * row;
+    const size_t att = !prompt_attn_fits(h) ? full
+        : attn_prompt_rows(cap, h.n_heads, h.n_kv_heads, h.d_head, h.max_ctx, prefill_split(h, true)) * row;
+    const size_t most = 4 * (size_t)cap * (h.d_model + 2 * (size_t)h.n_kv_heads * h.d_head) + full;
+    return std::min(std::max(att, prefill_part_floats(d)), most);
+}
+
 // Buffers of the prompt pass, in allocation order (mirrored by build_prefill).
 void plan_prefill(Plan &P, const cmolhip_model_desc_t *d)
 {
     const cmolhip_hparams_t &h = d->hp;
     const int cap = prefill_cap(h);
-    const int ms = attn_max_splits(h.max_ctx, prefill_split(h));
-    const size_t np = (size_t)h.n_kv_heads * ms * (h.n_heads / h.n_kv_heads);
     P.add((size_t)cap * 3 * 4);
     P.add((size_t)cap * 4);
     P.add((size_t)cap * h.d_model * 4);
@@ -999,12 +1016,9 @@ void plan_prefill(Plan &P, const cmolhip_model_desc_t *d)
     P.add(act_bytes(h.d_model, cap));
     P.add((size_t)cap * h.d_model * 4);
     P.add((size_t)cap * h.d_model * 4);
-    P.add((size_t)cap * np * 4);
-    P.add((size_t)cap * np * 4);
-    P.add((size_t)cap * np * h.d_head * 4);
     if (has_qk_norm(d)) P.add((size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head) * 4);
     if (prompt_attn_fits(h) && !h.kv_f16) P.add(attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx));
-    P.add(prefill_part_floats(d) * 4);
+    P.add(prefill_part_cap(d) * 4);
 }
 
 
@@ -1385,15 +1399,19 @@ int enqueue_prefill(cmolhip_model *m, Prefill &F, Batch &B, int n, bool last, hi
         at.kv_f16 = hp.kv_f16;
         at.split = F.split;
         at.max_splits = F.max_splits;
-        at.pm = F.pm;
-        at.pl = F.pl;
-        at.po = F.po;
+        at.po = F.part;
+        at.pm = F.part + F.part_rows * hp.d_head;
+        at.pl = at.pm + F.part_rows;
         at.out = nullptr;
         at.next = act_out(F.op_o, L.o.dtype, n, nullptr, nullptr, 0);
         // the pass's tokens share every K/V tile (flash style on MFMA); other
-        // shapes take the split kernels
-        if (prompt_attn_on() && launch_attn_prompt(at, F.kv_hl, F.h_steps[3 * (n - 1) + 2], st) == 0) {
-        } else {
+        // shapes, and a device that refuses the prompt kernel its LDS, take
+        // the split kernels, in as many splits as the partials have room for
+        if (!prompt_attn_on() || launch_attn_prompt(at, F.part_rows, F.kv_hl, F.h_steps[3 * (n - 1) + 2], st) != 0) {
+            while (at.max_splits > 1 && (size_t)n * hp.n_heads * at.max_splits > F.part_rows) {
+                at.split *= 2;
+                at.max_splits = attn_max_splits(hp.max_ctx, at.split);
+            }
             RC(launch_attn(at, st));
         }
 
@@ -1505,10 +1523,9 @@ int build_prefill(cmolhip_model *m, Prefill &F, size_t part_floats)
     cmolhip_ctx_t *c = m->ctx;
     const cmolhip_hparams_t &h = m->hp;
     F.cap = prefill_cap(h);
-    F.split = prefill_split(h);
+    F.split = prefill_split(h, prompt_attn_fits(h));
     F.max_splits = attn_max_splits(h.max_ctx, F.split);
     const int cap = F.cap;
-    const size_t np = (size_t)h.n_kv_heads * F.max_splits * (h.n_heads / h.n_kv_heads);
     RC(arena_get(c, (size_t)cap * 3, &F.steps));
     RC(arena_get(c, (size_t)cap, &F.slot_ids));
     RC(arena_get(c, (size_t)cap * h.d_model, &F.x));
@@ -1518,13 +1535,11 @@ int build_prefill(cmolhip_model *m, Prefill &F, size_t part_floats)
     for (int i = 0; i < 5; i++) RC(cmolhip_alloc(c, act_bytes(opk[i], cap), ALIGN, (void **)ops[i]));
     RC(arena_get(c, (size_t)cap * h.d_model, &F.ss_a));
     RC(arena_get(c, (size_t)cap * h.d_model, &F.ss_b));
-    RC(arena_get(c, (size_t)cap * np, &F.pm));
-    RC(arena_get(c, (size_t)cap * np, &F.pl));
-    RC(arena_get(c, (size_t)cap * np * h.d_head, &F.po));
     if (m->qk_norm) RC(arena_get(c, (size_t)cap * (h.d_model + 2 * h.n_kv_heads * h.d_head), &F.qkv_raw));
     if (prompt_attn_fits(h) && !h.kv_f16)
         RC(arena_get(c, attn_prompt_kv_bytes(h.n_kv_heads, h.d_head, h.max_ctx) / sizeof(_Float16), &F.kv_hl));
     F.part_cap = part_floats;
+    F.part_rows = part_floats / (h.d_head + 2);
     if (part_floats) RC(arena_get(c, part_floats, &F.part));
     HC(hipHostMalloc((void **)&F.h_steps, (size_t)cap * 3 * 4, hipHostMallocDefault));
     HC(hipHostMalloc((void **)&F.h_slots, (size_t)cap * 4, hipHostMallocDefault));
@@ -1786,7 +1801,7 @@ int build_model(cmolhip_model *m, const cmolhip_model_desc_t *d, const Plan &P)
     m->multi.reset(new Batch());
     RC(build_batch(m, *m->multi, multi_cap(h), batch_part_floats(d, multi_cap(h))));
     m->pf.reset(new Prefill());
-    RC(build_prefill(m, *m->pf, prefill_part_floats(d)));
+    RC(build_prefill(m, *m->pf, prefill_part_cap(d)));
     if (persist_format(d)) RC(build_persist(m, persist_format(d)));
     HC(hipStreamSynchronize(c->stream));
     if (m->use_graph) {

@@ -314,8 +314,11 @@ int launch_attn_merge_wave(const AttnArgs &a, hipStream_t s);
 // consecutive tokens of one session, d_head 64 / 128; returns -4 for shapes
 // it does not take (the caller runs launch_attn).  last = the pass's largest
 // seqlen.  kv_hl (fp32 caches only): attn_prompt_kv_bytes of scratch for the
-// high/low f16 copy of the session's cache positions 0 .. last-1.
-int launch_attn_prompt(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s);
+// high/low f16 copy of the session's cache positions 0 .. last-1.  part_rows:
+// room at a.po / pm / pl, in query heads x tokens x splits.
+int launch_attn_prompt(const AttnArgs &a, size_t part_rows, _Float16 *kv_hl, int last, hipStream_t s);
+// The most rows of partials a pass of up to cap tokens takes when given room.
+size_t attn_prompt_rows(int cap, int n_heads, int n_kv, int d_head, int max_ctx, int split);
 // (attn_prompt.hip)
 size_t attn_prompt_kv_bytes(int n_kv, int d_head, int max_ctx);
 

@@ -104,3 +104,33 @@ def test_scratch_planner_rejects_bad_shapes():
     out = C.c_size_t()
     assert L.cmolhip_batch_scratch_floats(C.byref(desc), 0, C.byref(out)) == native.CMOL_ERR_ARGS
     assert L.cmolhip_batch_scratch_floats(None, 4, C.byref(out)) == native.CMOL_ERR_ARGS
+
+
+# (layers, d_model, heads, kv heads, d_ffn, vocab, max_ctx, sessions, fp16 cache,
+# prompt chunk, layer format): device bytes that models of these shapes took
+# when a prompt's GEMMs split k into at most four ranges and prompts over fp16
+# caches ran the split attention kernels
+BYTES = {
+    (4, 2048, 16, 4, 11008, 128256, 4096, 1, 1, 512, Q4_0): 674789120,
+    (4, 2048, 16, 4, 11008, 128256, 16384, 1, 1, 2048, Q4_0): 1306318592,
+    (4, 2048, 16, 4, 11008, 128256, 16384, 1, 0, 2048, Q4_0): 1780274944,
+    (4, 2048, 16, 4, 11008, 128256, 330, 32, 1, 64, Q4_K): 684280832,
+    (8, 960, 15, 5, 2560, 49152, 1088, 16, 0, 512, Q5_0): 577294848,
+    (30, 576, 9, 3, 1536, 49152, 8192, 1, 1, 512, Q8_0): 417067520,
+    (4, 4096, 32, 8, 14336, 32000, 64, 1, 0, 512, Q4_0): 722589952,
+    (2, 256, 4, 2, 512, 1024, 4096, 4, 1, 64, Q8_0): 24181504,
+    (2, 512, 16, 4, 1024, 512, 4096, 1, 1, 512, Q8_0): 35100416,
+}
+
+
+@pytest.mark.parametrize("shape", BYTES)
+def test_a_model_takes_no_more_memory_than_it_did(shape):
+    """A model that just fits a device stays creatable: what the prompt passes
+    reserve is bounded by what they reserved before."""
+    nl, d, heads, kv, ffn, vocab, ctx, sessions, f16, chunk, dt = shape
+    hp = native.HParams(nl, heads, kv, d, d // heads, ffn, vocab, ctx, sessions, 4, f16, chunk, 1e4, 1e-6)
+    desc, keep = native.shape_desc(hp, *([dt] * 6), Q8_0)
+    need = C.c_size_t()
+    assert native.lib().cmolhip_model_plan(C.byref(desc), C.byref(need)) == 0
+    assert need.value <= BYTES[shape]
+    del keep
