@@ -89,7 +89,7 @@ __global__ __launch_bounds__(NWV * 64) void k_attn_h(AttnArgs a)
     const int cnt = min(L, t0 + a.split) - t0;
     const int nch = (cnt + CH - 1) / CH;
     const int nact = (L + a.split - 1) / a.split;
-    const size_t kvo = (size_t)(a.kv.slot_ids ? slot : n) * a.kv.slot_stride + a.kv.layer_off;
+    const size_t kvo = kv_offset_of(a.kv, n, slot);
     const size_t off = kvo + (size_t)kvh * a.max_ctx * DH + (size_t)t0 * DH;
     const uint8_t *kb = (const uint8_t *)((const KT *)a.kv.k_base + off);
     const uint8_t *vb = (const uint8_t *)((const KT *)a.kv.v_base + off);

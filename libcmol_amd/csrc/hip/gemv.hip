@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void k_gemv_b_finish(GemvArgs a, int splits, i
         s = wave_sum(s);
         nrm = 1.0f / sqrtf(s / (float)a.w.cols + a.in.eps);
     }
-    epi_pre_cs(a, EPI, row, act, pre);
+    epi_pre_cs(a, EPI, v, row, act, pre);
     // slices added in ascending order
     float y = 0.0f;
 #pragma unroll

@@ -199,12 +199,12 @@ __device__ __forceinline__ void epi_pre_load(const GemvArgs &a, int epi, int v, 
 
 // Second part, once the first part's loads have landed: the clamped
 // position, the cache offset, and the RoPE pair of the row.
-__device__ __forceinline__ void epi_pre_cs(const GemvArgs &a, int epi, int row, bool act, EpiPre &p)
+__device__ __forceinline__ void epi_pre_cs(const GemvArgs &a, int epi, int v, int row, bool act, EpiPre &p)
 {
     if (act && epi == EPI_QKV) {
         const int pos = a.pos ? p.pos : a.pos0;
         p.pos = min(max(pos, 0), a.max_ctx - 1);
-        p.kvo = (a.kv.slot_ids ? (size_t)p.slot * a.kv.slot_stride : 0) + a.kv.layer_off;
+        p.kvo = kv_offset_of(a.kv, v, p.slot);
         p.cs = rope_cs(a, row + a.row_base, p.pos);
     }
 }
@@ -412,7 +412,7 @@ void k_gemv(GemvArgs a, GemvShape sh)
     __builtin_amdgcn_s_waitcnt(WAITCNT_VM_LGKM0(LPS * U));
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    epi_pre_cs(a, epi, prow, pact, pre);
+    epi_pre_cs(a, epi, v0 + pv, prow, pact, pre);
 
     // A-operand row fed by this lane per group: LDS address of block 0 and
     // per-block stride (rows beyond 2nF read the zero slot)

@@ -116,17 +116,20 @@ __device__ __forceinline__ void mfma_block(f32x4 &acc, const f16x8 &xv, const f1
 // KV caches of one layer for a batch of activation vectors: vector n uses
 // slot slot_ids[n], whose K cache starts at k_base + slot*slot_stride +
 // layer_off elements (fp32 or fp16 per kv_f16); without slot_ids (decode
-// attention calls) vector n uses slot n.
+// attention calls) vector n uses slot n, in every kernel.
 struct KVRef {
     void *k_base, *v_base;
     size_t slot_stride, layer_off;
     const int32_t *slot_ids;
 };
 
-__device__ inline size_t kv_offset(const KVRef &r, int n)
+// slot: slot_ids[n] (not looked at without slot_ids)
+__device__ inline size_t kv_offset_of(const KVRef &r, int n, int slot)
 {
-    return (size_t)(r.slot_ids ? r.slot_ids[n] : n) * r.slot_stride + r.layer_off;
+    return (size_t)(r.slot_ids ? slot : n) * r.slot_stride + r.layer_off;
 }
+
+__device__ inline size_t kv_offset(const KVRef &r, int n) { return kv_offset_of(r, n, r.slot_ids ? r.slot_ids[n] : 0); }
 
 // ---------------------------------------------------------------------------
 // Activation operands.
