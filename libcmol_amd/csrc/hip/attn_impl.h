@@ -926,9 +926,11 @@ __device__ inline int wave_scan_i(int v)   // inclusive prefix sum over the lane
     }
     return v;
 }
+// (a length below 0 is no context, as on the split grid: taken as it is, it
+// would move the line offsets of the contexts behind it, out of the partials)
 __device__ __forceinline__ int attn_len(const AttnArgs &a, int i)
 {
-    return i < a.n ? min(a.seqlen[i * a.seqlen_stride], a.max_ctx) : 0;
+    return i < a.n ? max(min(a.seqlen[i * a.seqlen_stride], a.max_ctx), 0) : 0;
 }
 // Line length and range length of the balanced walk; every wave computes
 // them (no barrier), the attention and merge kernels alike.  l0: this

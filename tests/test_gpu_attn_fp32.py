@@ -61,3 +61,32 @@ def test_fp32_balanced_equals_split_grid_closely(ctx, gpu, monkeypatch):
         outs.append(ctx.d2h(dout, q.shape, np.float32))
     for o in outs[1:]:
         assert np.allclose(outs[0], o, rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("kv_f16", [0, 1])
+def test_contexts_without_positions_change_no_other(ctx, gpu, monkeypatch, kv_f16):
+    """Lengths of zero and below among others, on balanced ranges: those
+    contexts' outputs stay as they were, the others equal a call without them."""
+    n_heads, n_kv, d_head, max_ctx = 16, 4, 128, 1024
+    lens = [700, -900, 0, 1024, -1, -(1 << 31), 300]
+    real = [i for i, m in enumerate(lens) if m > 0]
+    rng = np.random.default_rng(11)
+    n = len(lens)
+    q = rng.standard_normal((n, n_heads * d_head)).astype(np.float32)
+    kc, vc = (rng.standard_normal((n, n_kv, max_ctx, d_head)).astype(np.float16 if kv_f16 else np.float32)
+              for _ in range(2))
+    monkeypatch.setenv("CMOL_ATTN_BAL", "200")
+
+    def run(rows):
+        m = len(rows)
+        out = np.full((m, n_heads * d_head), 7.0, np.float32)
+        dq, dk, dv, dout = ctx.upload(q[rows]), ctx.upload(kc[rows]), ctx.upload(vc[rows]), ctx.upload(out)
+        ds = ctx.upload(np.array([lens[i] for i in rows], np.int32))
+        gpu.check(gpu.lib().cmolhip_attn_decode(ctx.h, m, *(C.c_void_p(p) for p in (dq, dk, dv, ds)), n_heads, n_kv,
+                                                d_head, max_ctx, kv_f16, 64, C.c_void_p(dout)), "attn")
+        return ctx.d2h(dout, out.shape, np.float32)
+
+    got, want = run(list(range(n))), run(real)
+    # fp32 sums over ranges cut elsewhere
+    assert np.allclose(got[real], want, rtol=1e-5, atol=1e-6)
+    assert (got[[i for i in range(n) if i not in real]] == 7.0).all()
