@@ -27,7 +27,10 @@
 // times 2^-11 against the low part times 2^11), so one scale FMA per output
 // and block serves both.
 #pragma once
+#include "gemm_slices.h"
 #include "gemv_impl.h"
+
+#include <algorithm>
 
 // Adds the ks k ranges' partial sums of a prompt GEMM in order, applies the
 // RMSNorm factor and runs the epilogue (gemv.hip).
@@ -43,7 +46,7 @@ struct GemmShape {
     int mt;          // vector tiles (GEMM_BM vectors each)
     int nt;          // 128-row tiles
     int ga;          // XCD slices along the vector tiles (1, 2, 4, 8)
-    int mts, nts;    // vector / row tiles per slice
+    int mts, nts;    // vector / row tiles per slice (gemm_slices.h)
     int ks, kq;      // k ranges (grid.y) of kq block quads each; ks > 1: fp32 partial sums to a.part
     int fq;          // > 0: after fq quads (even) of its range a work-group sets its sums aside in LDS
 };
@@ -515,12 +518,10 @@ int launch_gemm_dt(const GemvArgs &a, int epi, hipStream_t s)
     sh.kq = (KQ + ks - 1) / ks;
     sh.mt = (a.n + GEMM_BM - 1) / GEMM_BM;
     sh.nt = (a.w.rows + GEMM_BN - 1) / GEMM_BN;
-    // one slice of vector tiles per XCD (at 2048 vectors: 256 KiB of operand
-    // per 32-vector tile, eight per XCD) unless there are fewer vector tiles
-    sh.ga = 8;
-    while (sh.ga > 1 && sh.ga > sh.mt) sh.ga >>= 1;
-    sh.mts = (sh.mt + sh.ga - 1) / sh.ga;
-    sh.nts = (sh.nt + 8 / sh.ga - 1) / (8 / sh.ga);
+    const GemmSlices sl = gemm_slices(sh.mt, sh.nt, ks, sh.kq, std::max(1, gemv_cus() / 8));
+    sh.ga = sl.ga;
+    sh.mts = sl.mts;
+    sh.nts = sl.nts;
     const long wgs = 8L * sh.mts * sh.nts;
     if (wgs > 0x7fffffffL) return -6;
     // fewer than four work-groups per CU (the grids that two ranges of twice

@@ -76,6 +76,16 @@ def test_gemm_k_ranges_match_oracle(gpu, dtype, rows, cols, fold, n, norm):
     ctx.close()
 
 
+# vector tiles that do not divide by eight, in one, two and four slices per the
+# grid's row tiles, the last row tile ragged; split k and not
+@pytest.mark.parametrize("rows,cols,n", [(2500, 256, 160), (2500, 256, 188), (2500, 256, 300), (5000, 128, 350),
+                                         (2500, 512, 600), (520, 4096, 188)])
+def test_gemm_slices_match_oracle(gpu, rows, cols, n):
+    ctx = gpu.Ctx(512 << 20)
+    check_gemm(ctx, 2, rows, cols, 1, n, True)
+    ctx.close()
+
+
 def test_gemm_small_arena_takes_fewer_ranges(gpu):
     """An arena with room for fewer k ranges' partial sums than the product
     would take: the call still runs, on fewer ranges."""
