@@ -115,30 +115,24 @@ __global__ __launch_bounds__(256) void k_kv_hilo(AttnArgs a, int last, _Float16 
     }
 }
 
-// Takes the values that are not finite out of the V part `v` of a half's
-// staged tile, by the half's 256 threads (t) and within two barriers of the
-// work-group: they become 0 and bad[position] is set.  `on`: the half has a tile
-// with masked positions.
+// Takes the V values that are not finite out of a half's staged tile, by the
+// half's 256 threads (t) before a barrier of the work-group: they become 0, and
+// the first value of their position's K row NaN, so that the rows that see the
+// position have its weight NaN (the others mask its score).  `on`: the half has
+// a tile with masked positions.
 template <int DH, bool F16>
-__device__ __forceinline__ void pa_take_apart(uint8_t *v, uint8_t *bad, int t, bool on)
+__device__ __forceinline__ void pa_take_apart(uint8_t *k, uint8_t *v, int t, bool on)
 {
-    constexpr int TP = F16 ? 64 : KVT_POS, CHUNKS = TP * DH * 2 / 16;   // 16-byte pieces (fp32: high ones)
-    if (t < TP) bad[t] = 0;
-    __syncthreads();
-    for (int q = t; on && q < CHUNKS; q += 256) {
-        // fp32: piece (dimension tile, lane), its high half here and its low one 1 KiB on
-        f16x8 *p = (f16x8 *)(v + (F16 ? q * 16 : (q >> 6) * 2048 + (q & 63) * 16));
-        f16x8 x = *p;
-        bool any = false;
-        for (int e = 0; e < 8; e++) {
-            if ((__builtin_bit_cast(uint16_t, (_Float16)x[e]) & 0x7c00) != 0x7c00) continue;
-            const int g = (q & 63) >> 4;
-            bad[F16 ? q * 16 / (2 * DH) : 4 * g + (e & 3) + 16 * (e >> 2)] = 1;
-            x[e] = 0;
-            if (!F16) ((_Float16 *)p)[512 + e] = 0;
-            any = true;
-        }
-        if (any) *p = x;
+    constexpr int TP = F16 ? 64 : KVT_POS, KS = DH / 32;
+#pragma unroll 1
+    for (int q = t; on && q < TP * DH; q += 256) {
+        // fp32: high piece q / 512, lane (q % 512) / 8, the low one 512 halves on
+        uint16_t *p = (uint16_t *)v + (F16 ? q : (q >> 9) * 1024 + (q & 511));
+        if ((*p & 0x7c00) != 0x7c00) continue;
+        *p = 0;
+        if (!F16) p[512] = 0;
+        const int pos = F16 ? q / DH : 4 * ((q >> 7) & 3) + (q & 3) + 16 * ((q >> 2) & 1);
+        *(uint16_t *)(k + (pos >> 4) * KS * (F16 ? 1024 : 2048) + (pos & 15) * 16) = 0x7e00;
     }
     __syncthreads();
 }
@@ -158,7 +152,6 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
     constexpr int PIECES = TILE / 1024 / 4;           // fp32: pieces per wave
     constexpr int DH2 = DT / 2;                       // dimension tiles each half finishes
     extern __shared__ __attribute__((aligned(256))) uint8_t smem_p[];   // [stage][half][TILE]
-    __shared__ uint8_t badrow[2][TP];   // V rows of the halves' tiles that are not finite (see apart)
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, col = lane & 15;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), half = wid >> 2, w4 = wid & 3;
@@ -258,9 +251,10 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
             __builtin_amdgcn_s_waitcnt(WAITCNT_VM_LGKM0(0));
             __syncthreads();
             if (p0 + 2 * TP < pb) issue(st ^ 1, p0 + 2 * TP);
-            if (__builtin_expect(apart && pp + 2 * TP > whole, 0))   // (alike in both halves: it has barriers)
-                pa_take_apart<DH, F16>(smem_p + (st * 2 + half) * TILE + KB, badrow[half], tid & 255,
-                                       p0 < pb && p0 + TP > whole);
+            if (__builtin_expect(apart && pp + 2 * TP > whole, 0)) {   // (alike in both halves: it has a barrier)
+                uint8_t *k = smem_p + (st * 2 + half) * TILE;
+                pa_take_apart<DH, F16>(k, k + KB, tid & 255, p0 < pb && p0 + TP > whole);
+            }
             if (p0 >= pb) continue;          // (the last pair may be one tile)
             const uint8_t *ks_ = smem_p + (st * 2 + half) * TILE, *vs_ = ks_ + KB;
             // ---- scores: sc[c][i] = position p0 + 16c + 4g + i of this lane's row
@@ -291,13 +285,6 @@ void k_attn_prompt(AttnArgs a, const _Float16 *hl, int tiles)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
                         if (p0 + 16 * c + 4 * g + i >= lim) sc[c][i] = -INFINITY;
-                if (__builtin_expect(apart, 0)) {
-#pragma unroll
-                    for (int c = 0; c < CT; c++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            if (badrow[half][16 * c + 4 * g + i] && p0 + 16 * c + 4 * g + i < lim) sc[c][i] = __builtin_nanf("");
-                }
             }
             // ---- online softmax of the row (its scores: lanes col + 16 g) ----
             float mx = sc[0][0];
