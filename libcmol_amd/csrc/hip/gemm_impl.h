@@ -10,7 +10,8 @@
 // pipeline: the activation operand of quad kk+1 is copied into LDS with
 // direct-to-LDS loads and each wave loads the weight codes of its two
 // virtual tiles for it into registers while quad kk is contracted.  32 KiB
-// of LDS and 128 VGPRs keep four work-groups on a CU, each with its own
+// of LDS (40 or 48 where a range is summed in two halves, see launch_gemm_dt)
+// and 128 VGPRs keep four work-groups on a CU (three at 48), each with its own
 // barrier.  Eight-wave 64 x 128 tiles (two work-groups per CU, half the weight
 // decoding per product) took, Q4_0 11008 inputs x 2048 rows / 2048 x 22016:
 // 2048 vectors 211 / 417 us against 216 / 406, 1500 vectors 192 / 321 against
@@ -48,7 +49,7 @@ struct GemmShape {
     int ga;          // XCD slices along the vector tiles (1, 2, 4, 8)
     int mts, nts;    // vector / row tiles per slice (gemm_slices.h)
     int ks, kq;      // k ranges (grid.y) of kq block quads each; ks > 1: fp32 partial sums to a.part
-    int fq;          // > 0: after fq quads (even) of its range a work-group sets its sums aside in LDS
+    int fq;          // > 0: after fq quads (even) of its range a work-group sets its sums aside
 };
 
 // acc += the block's contribution for 16 vectors: xh holds their high
@@ -249,8 +250,8 @@ __device__ __forceinline__ void epi_runs(const GemvArgs &a, Src src, int m0, int
 // Held to four waves per SIMD (128 VGPRs).  Unheld, the Q8_0 and K-quant
 // instances took 129-160 and ran half the work-groups: 22016 x 2048 at 2048
 // vectors, Q8_0 590 -> 462 us, Q4_K 822 -> 612 (4 VGPRs spilled), Q6_K 1031
-// -> 791 (14 spilled).
-template <int DT>
+// -> 791 (18 spilled).
+template <int DT, bool SLIM>
 __global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm(GemvArgs a, GemmShape sh)
 {
     constexpr int HG = 2, NJ = 2;                 // vector groups and virtual tiles per wave
@@ -394,14 +395,21 @@ __global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) vo
     // the body is unconditional (steps past the end compute nothing and
     // re-read the last quad) so every wait count is the same on each pass
     const bool halves = sh.fq && kb + sh.fq < ke;
-    f32x4 *aside = (f32x4 *)(smem + GEMM_STAGES * ASTAGE) + tid;   // [HG NJ][threads], each thread its own
+    // the first half's sums: [HG NJ][threads] in LDS, each thread its own;
+    // SLIM: those of the last vector group in registers
+    constexpr int HL = SLIM ? HG - 1 : HG;
+    f32x4 *aside = (f32x4 *)(smem + GEMM_STAGES * ASTAGE) + tid;
+    f32x4 keep[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) keep[j] = zero4;
     for (int k0 = kb; k0 < ke; k0 += GEMM_STAGES) {
         if (halves && k0 == kb + sh.fq) {
 #pragma unroll
             for (int h = 0; h < HG; h++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
-                    aside[(h * NJ + j) * GEMM_NT] = acc[h][j];
+                    if (h < HL) aside[(h * NJ + j) * GEMM_NT] = acc[h][j];
+                    else keep[j] = acc[h][j];
                     acc[h][j] = zero4;
                 }
         }
@@ -432,7 +440,7 @@ __global__ __launch_bounds__(GEMM_NT) __attribute__((amdgpu_waves_per_eu(4))) vo
         unsigned long long key[4] = {};   // EPI_LOGITS: the lane's best row per vector
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            if (halves) acc[h][j] += aside[(h * NJ + j) * GEMM_NT];
+            if (halves) acc[h][j] += h < HL ? aside[(h * NJ + j) * GEMM_NT] : keep[j];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int rl = (wid * NJ + j) * 16 + cl, row = nt_ * BN + rl;
@@ -528,14 +536,28 @@ int launch_gemm_dt(const GemvArgs &a, int epi, hipStream_t s)
     // the work would also serve): each range is summed in two halves, so a
     // range costs no precision against two of half its length (2048 inputs:
     // 1.39e-7 of the result in 2-norm, 1.69e-7 in one chain; 20.2 us against
-    // 19.7 at 2048 x 2048 x 512 vectors).  The 16 KiB of LDS it takes would
-    // cost fuller grids a fourth work-group per CU.
+    // 19.7 at 2048 x 2048 x 512 vectors).  Fuller grids run in one chain: the
+    // first half's sums, 16 KiB of LDS, would leave a CU three work-groups of
+    // four.
     sh.fq = (long)sh.mt * sh.nt * ks < 4L * gemv_cus() ? 2 * ((sh.kq + 3) / 4) : 0;
-    const size_t lds = (size_t)GEMM_STAGES * 4 * 4 * 2 * GEMM_BM * 16 + (sh.fq ? (size_t)GEMM_NT * 64 : 0);
+    // where that already makes a second round, with more than three work-groups
+    // per CU on the fullest XCD, half of those sums stay in registers instead.
+    // us, all in LDS / half: Q4_0 22016 x 2048 x 160 47.4 / 45.1, 5120 x 2048 x
+    // 700 49.4 / 46.0; Q4_K 2048 x 2048 x 1600 68.0 / 61.1; Q6_K (24 VGPRs
+    // spilled) 4096 x 4096 x 800 161 / 150.  Grids of one vector tile, bound by
+    // their weights, and several k ranges gain only in the formats that it makes
+    // spill nothing (128256 x 2048 x 17: Q4_0 49.4 / 46.8, Q5_0 63.2 / 61.7, Q8_0
+    // 55.5 / 56.8, Q6_K 93.9 / 96.2; 2048 x 11008 x 224, eight ranges: Q4_0 42.1
+    // / 39.6, Q4_K 52.7-53.7 / 54.0-54.5).
+    constexpr bool spills = DT != DT_Q4_0 && DT != DT_Q5_0;
+    const bool slim = sh.fq && (long)sh.mts * sh.nts * ks > 3L * (gemv_cus() / 8) && (!spills || (sh.mt > 1 && ks == 1));
+    const size_t lds = (size_t)GEMM_STAGES * 4 * 4 * 2 * GEMM_BM * 16 + (sh.fq ? (size_t)GEMM_NT * (slim ? 32 : 64) : 0);
     const dim3 grid((unsigned)wgs, (unsigned)ks), block(GEMM_NT);
-    if (a.ev_start)
-        hipExtLaunchKernelGGL((k_gemm<DT>), grid, block, lds, s, a.ev_start, ks > 1 ? nullptr : a.ev_stop, 0, a, sh);
-    else
-        hipLaunchKernelGGL((k_gemm<DT>), grid, block, lds, s, a, sh);
+    auto go = [&](auto kern) {
+        if (a.ev_start) hipExtLaunchKernelGGL(kern, grid, block, lds, s, a.ev_start, ks > 1 ? nullptr : a.ev_stop, 0, a, sh);
+        else hipLaunchKernelGGL(kern, grid, block, lds, s, a, sh);
+    };
+    if (slim) go(k_gemm<DT, true>);
+    else go(k_gemm<DT, false>);
     return ks > 1 ? launch_gemm_finish(a, epi, ks, s) : 0;
 }

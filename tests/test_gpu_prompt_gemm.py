@@ -86,6 +86,18 @@ def test_gemm_slices_match_oracle(gpu, rows, cols, n):
     ctx.close()
 
 
+# three to four work-groups per CU, whose first half's sums are kept half in
+# registers: 10 vector tiles x 101 row tiles, the last ragged, and a single
+# vector tile (there only the formats that spill nothing); five quads, so the
+# second half is the shorter one
+@pytest.mark.parametrize("dtype,cols", [(2, 640), (6, 640), (8, 640), (12, 768), (14, 768)])
+@pytest.mark.parametrize("rows,n", [(12805, 300), (125000, 20)])
+def test_gemm_kept_sums_match_oracle(gpu, dtype, cols, rows, n):
+    ctx = gpu.Ctx(1 << 30)
+    check_gemm(ctx, dtype, rows, cols, 1, n, n == 300)
+    ctx.close()
+
+
 def test_gemm_small_arena_takes_fewer_ranges(gpu):
     """An arena with room for fewer k ranges' partial sums than the product
     would take: the call still runs, on fewer ranges."""
