@@ -3,6 +3,7 @@ every entry point its headers declare; public utilities and load-time error
 paths behave like the reference's (src/api.c:24-41,139-206,356-398)."""
 import ctypes as C
 import os
+import resource
 import re
 import struct
 
@@ -182,14 +183,20 @@ def test_scheduler_window_gathers_returning_callers():
 
 
 def test_scheduler_posts_wake_no_waiter_early():
-    """32 callers, a short window and long device steps: a posted step must
-    not wake the other waiters (each would re-check, and a leader woken
-    before the set is complete runs a partial batch). Batches stay near the
-    step count of the longest-lived caller (91 here); waking every waiter on
-    each post gave about 160."""
+    """32 callers and a window that outlasts their return: a posted step must
+    not wake the other waiters (each would take the lock, re-check and wait
+    again).  Batches stay near the step count of the longest-lived caller (91
+    here), and a caller's step costs at most one voluntary context switch each
+    for its wait, for the lock behind it and for the lock of its next post,
+    with the leader's sleep below four; waking every waiter on each post takes
+    about nine.  (Counted rather than timed: with a window of 200 us the batch
+    count told the two apart only where 32 threads wake up within it.)"""
     threads, steps = 32, 60
     st = np.zeros(3, np.uint64)
-    assert native.lib().cmol__sched_selftest(threads, steps, 200, 4500, 0, native.ptr(st)) == 0
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_nvcsw
+    assert native.lib().cmol__sched_selftest(threads, steps, 20000, 300, 0, native.ptr(st)) == 0
+    switches = resource.getrusage(resource.RUSAGE_SELF).ru_nvcsw - before
     batches, total = int(st[0]), int(st[1])
     assert total == sum(steps + i for i in range(threads))
     assert batches <= steps + threads - 1 + 25
+    assert switches <= 4 * total
