@@ -16,9 +16,10 @@ ATOL, RTOL = 1e-4, 1e-3
 # widths that end inside a 128-row tile (576 = 4.5, 320 = 2.5), a q|k|v row
 # count with heads of 64 and of 32, and a feed-forward width of odd blocks
 # (1056: 2112 interleaved rows = 16.5 tiles; 2080: the down projection also
-# splits k)
-@pytest.mark.parametrize("wtype", [synth.Q4_0, synth.Q5_0, synth.Q8_0])
-@pytest.mark.parametrize("heads,kv,d_model,d_ffn", [(9, 3, 576, 1056), (10, 2, 320, 2080)])
+# splits k); the K-quants, whose widths are whole tiles
+@pytest.mark.parametrize("wtype,heads,kv,d_model,d_ffn", [
+    (w, *shape) for shape in [(9, 3, 576, 1056), (10, 2, 320, 2080)] for w in (synth.Q4_0, synth.Q5_0, synth.Q8_0)
+] + [(synth.Q4_K, 12, 4, 768, 1792), (synth.Q6_K, 12, 4, 768, 1792)])
 @pytest.mark.parametrize("n", [9, 17, 33, 64, 65, 129])
 def test_prompt_epilogues_match_oracle(gpu, model_dir, wtype, heads, kv, d_model, d_ffn, n):
     spec = synth.ModelSpec(2, d_model, heads, kv, d_ffn, 512, ctx_len=192, wtype=wtype, embd_type=wtype, wstd=0.05,
