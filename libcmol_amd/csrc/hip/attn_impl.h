@@ -707,7 +707,7 @@ __device__ __forceinline__ void attn_piece_mfw(const AttnArgs &a, int kvh, int n
 // 512..4096 positions at 16/4 heads of 128, 227 MB, 41.4 us (5.5 TB/s) where
 // the split grid (attn.hip, k_attn_h: a 64-position split per 512-thread
 // work-group, one per CU by its LDS) took 85.5; 8 contexts of 64..4096 22.2 ->
-// 13.2 us.
+// 13.0 us.
 template <int DH, typename M>
 __device__ __forceinline__ void attn_piece_fw(const AttnArgs &a, int kvh, int n, int t0, int cnt, bool single,
                                               size_t sbase, size_t kvo)
@@ -943,7 +943,7 @@ __device__ __forceinline__ int attn_bal_range(const AttnArgs &a, int l0)
     const int line = wave_sum_i(t);
     // fp32: two steps of the work-group at least, or starting and merging the
     // pieces outweighs them (16/4 heads of 128, 8 contexts of 64..4096: ranges
-    // of 64 positions 15.2 + 5.7 us, of 128 13.2 + 4.6)
+    // of 64 positions 15.2 + 5.7 us, of 128 13.0 + 4.5)
     return max(a.kv_f16 ? a.split : max(a.split, 128), (line + a.bal - 1) / a.bal);
 }
 

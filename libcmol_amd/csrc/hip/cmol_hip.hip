@@ -367,8 +367,9 @@ static size_t product_part_floats(const cmolhip_qtensor_t &w, int n, bool norm)
 }
 
 // dy[n][rows] = W . op for a prepared operand: up to 32 vectors stream the
-// weights once through the matvec (k-split partial sums in part, part_cap
-// floats), more run the tiled MFMA GEMM.
+// weights through the matvec (9..32 over wide or large matrices through the
+// GEMM, batch_by_gemm), more run the tiled MFMA GEMM; partial sums of k ranges
+// in part, part_cap floats.
 static int launch_product(cmolhip_ctx_t *c, const cmolhip_qtensor_t *w, const void *op, int n,
                           const float *ss, float eps, float *dy, float *part, size_t part_cap,
                           void *ev_start, void *ev_stop)

@@ -145,7 +145,7 @@ __device__ __forceinline__ void gemm_norms(const GemvArgs &a, int m0, float *s_n
 // pairs), 16 lanes along a vector's rows.  The stores bound these epilogues:
 // one lane per row and 2-byte operand stores took 571 us for the gate/up
 // projection of 2048 tokens (22016 x 2048 Q4_0) where the same product with
-// plain stores takes 431; 479 with 16-byte ones (and gemm_norms).
+// plain stores took 431; 470-479 (400) with 16-byte ones and gemm_norms.
 // Rows come in whole operand blocks (RESID, SWIGLU: the consumer's inputs)
 // or whole 16-row heads (QKV).
 template <int EPI, int BM, int BR, int NT, typename Src>

@@ -55,7 +55,12 @@ size_t act_bytes(int K, int n)
 // 20.1 / 18.9 with the weights in the caches, but 22.0 / 22.5 with the
 // preparation and weights from HBM) or above 2^24 (Q6_K: 11008 x 2048 29.8 /
 // 23.8, 2048 x 5632 15.8 / 16.1); up to 16 vectors from two tiles per CU on (16
-// vectors Q8_0 49152 x 2048 27.9 / 29.6, 65536 x 2048 32.4 / 30.9).
+// vectors Q8_0 49152 x 2048 27.9 / 29.6, 65536 x 2048 32.4 / 30.9).  Narrow
+// heads above 16 vectors (17): Q8_0 49152 x 576 17.5 / 13.8, Q5_0 49152 x 960
+// 28.4 / 19.9.  Inside lock-step steps of four 3B blocks (fp16 caches), with
+// the SwiGLU and residual epilogues, the same order: all matrices Q4_K, 17
+// sessions 410 / 397, 24 427 / 412, 32 474 / 442; Q6_K 550 / 491, 568 / 513,
+// 612 / 527.
 static bool batch_by_gemm(const QTensor &w, int n)
 {
     // (folded tensors serve one session; the GEMM's weight offsets are 32-bit)
