@@ -56,7 +56,7 @@
 // block's work grows with its position, so the longest prefixes start first.
 // With four waves per work-group (one tile at a time, every block of a
 // 2048-token pass resident at once) a pass lasted as long as its longest
-// block.  Per layer at 16/4 heads of 128, 2048 tokens over fp32: 116 -> 78-88
+// block.  Per layer at 16/4 heads of 128, 2048 tokens over fp32: 116 -> 73-88
 // us.  Over fp16, where such passes ran the decode split kernel (one
 // work-group per token): 512 tokens behind 1300 positions 314 + 17 us (merge)
 // -> 31 + 6, 188 behind 1812 120 + 8 -> 20 + 5.  Work-groups of 128 query
