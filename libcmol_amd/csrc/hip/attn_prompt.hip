@@ -454,7 +454,10 @@ static int launch_dh(const AttnArgs &a, _Float16 *kv_hl, int last, hipStream_t s
         return hipFuncSetAttribute((const void *)k_attn_prompt<DH, F16>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) ==
                hipSuccess;
     });
-    if (!ok) return -4;
+    if (!ok) {
+        (void)hipGetLastError();   // (not the split kernels' launch error)
+        return -4;
+    }
     const int QT = 64 / (a.n_heads / a.n_kv);
     const int tiles = (a.max_ctx + KVT_POS - 1) / KVT_POS;
     if constexpr (!F16)
